@@ -881,13 +881,6 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
     return 0;
 }
 
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // One work unit, phases A-D.  It and the stages it calls (generation, both
 // sweeps, the line map) are inlined into the kernel: a call would take the
 // frame, the scene descriptor and the queues by address, which keeps them in
@@ -940,7 +933,7 @@ __device__ __forceinline__ void adj_unit(const Frame &f, const AdjDesc &d, int l
     // optional phase clocks (wave-uniform points): [0] A generate [1] A sort
     // [2] A sweep [3] B generate [4] B sort [5] B sweep [6] C [7] units
     unsigned long long *clk = f.stage_cycles;
-    uint16_t *hist = reinterpret_cast<uint16_t *>(&tt->gc[0][0][0]) + lane;   // sort histogram
+    uint16_t *hist = reinterpret_cast<uint16_t *>(&tt->sec) + lane;   // sort histogram
     long long tclk = clk ? clock64() : 0;
     auto stamp = [&](int i) {
         if (!clk) return;
@@ -979,7 +972,7 @@ __device__ __forceinline__ void adj_unit(const Frame &f, const AdjDesc &d, int l
         fq.head = q.head;
         fq.len = q.len;
     }
-    if (ok) status = sweep_forward<kCompact>(f, d, fq, c, Stack{s0, s1, 0u}, sidx, tt, loss);
+    if (ok) status = sweep_forward<kCompact>(f, d, fq, c, Stack{s0, s1}, sidx, tt, loss);
     stamp(2);
     q.spilled = q.spilled || fq.spilled;
     if (active && (q.overflow || fq.overflow)) status |= kStatusOverflow;
@@ -995,7 +988,7 @@ __device__ __forceinline__ void adj_unit(const Frame &f, const AdjDesc &d, int l
     ok = active && !q.spilled && !q.overflow;
     if (ok && !copied) radix_sort_queue(q, hist, s.sort_bits, c.float_height);
     stamp(4);
-    if (ok) status = sweep_backward<kCompact>(f, d, q, c, Stack{s0, s1, 0u}, sidx, tt, straight, dcol, orig);
+    if (ok) status = sweep_backward<kCompact>(f, d, q, c, Stack{s0, s1}, sidx, tt, straight, dcol, orig);
     stamp(5);
     // B repeats A's queue operations on the same records, so it cannot
     // outgrow a ring the forward sweep fit in; should it, the unit goes to

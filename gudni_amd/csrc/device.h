@@ -610,16 +610,11 @@ enum Cross { kCrossRight, kCrossLeft, kCrossDown };
 
 struct Stack {
     uint64_t s0, s1;
-    uint32_t dirty;   // colour groups touched since their composite was cached
-    // a bit's colour group is (b * gm) >> 16, gm = ceil(2^16 / the group
-    // width) (TileTable::gm; exact for b < 128); 2048: groups of 32
-    uint32_t gm = 2048u;
     __device__ __forceinline__ void flip(uint32_t h)
     {
         const uint32_t b = h & kLabelMask;
         if (b < 64u) s0 ^= 1ull << b;
         else s1 ^= 1ull << (b - 64u);
-        dirty |= 1u << ((b * gm) >> 16);
     }
     // Crossing record h: an even-odd shape flips its bit (passHeader,
     // Kernels.cl:298-304).  A nonzero-fill shape adds the crossing's winding
@@ -649,7 +644,6 @@ struct Stack {
         const uint64_t m = 1ull << (b & 63u);
         uint64_t &word = b < 64u ? s0 : s1;
         word = v != 0 ? (word | m) : (word & ~m);
-        dirty |= 1u << ((b * gm) >> 16);
     }
 };
 
@@ -871,26 +865,34 @@ __device__ __forceinline__ float4 read_color(const SceneDesc &s, uint64_t tag, i
     return read_color_sub(s, tag, s.substances[tag & kTagIdMask], ax, ay);
 }
 
+// A wave's list of sections waiting for their colours: per section its area
+// (adj) and the stack it lies under, which the colour pass replaces by colour
+// x area.  info: the lane that swept it (bits 0..5), its pixel's row in that
+// lane's segment (6..18), whether it is its pixel's last (kSecEnd), and the
+// lane's next section in the list (24..31, kSecNone: none).
+constexpr int kSections = 192;             // three full waves of colours
+constexpr uint32_t kSecEnd = 1u << 19, kSecNone = 0xFFu;
+struct SectionList {
+    float4 val[kSections];
+    float adj[kSections];
+    uint32_t info[kSections];
+};
+
 // Per-wave LDS table of a compact tile's shapes by tile-local index: tag,
 // and the solid colour (in the coverage mode's form) or, for a picture or
 // gradient, the substance record itself.
 struct TileTable {
     uint64_t tag[128];
     float4 color[128];
-    // grouped colours (accurate mode): per lane, the premultiplied composite
-    // of each group of 32 tile-local shapes, [group][component][lane]
-    float gc[4][4][64];
+    SectionList sec;       // before the sweep: the sort's histogram
     uint64_t pic0, pic1;   // tile-local shapes whose substance is a picture
     int grouped;           // the tile qualifies for grouped colours
     // colour group g holds tile-local shapes [g gq, (g+1) gq), gq = ceil(n / 4)
-    // for a tile of n shapes; gm = ceil(2^16 / gq) maps a shape to its group
-    uint32_t gq, gm;
-    // per group: the tile-local shapes some lane of the current unit holds a
-    // record or an enclosure of, i.e. every stack bit it can set
-    uint32_t cand[4];
+    // for a tile of n shapes
+    uint32_t gq;
 };
-static_assert(sizeof(TileTable::gc) >= sizeof(uint16_t) * kWave * (1 << kRadixMaxBits),
-              "the sort histogram lives in the colour cache");
+static_assert(sizeof(SectionList) >= sizeof(uint16_t) * kWave * (1 << kRadixMaxBits),
+              "the sort histogram lives in the section list");
 
 // Bits [start, start + q) of the 128-bit set (s1:s0), q <= 32, start < 128;
 // bits past 127 read as 0.
@@ -903,19 +905,31 @@ __device__ __forceinline__ uint32_t group_bits(uint64_t s0, uint64_t s1, uint32_
     return (uint32_t)v & (q >= 32u ? 0xFFFFFFFFu : ((1u << q) - 1u));
 }
 
+// OR of a word over the wave's 64 lanes (all of them active).
+__device__ __forceinline__ uint32_t wave_or(uint32_t v)
+{
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);   // row_shr:1
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);   // row_shr:2
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);   // row_shr:4
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);   // row_shr:8
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, true);   // row_bcast:15
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, true);   // row_bcast:31
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // Composite of one group's set shapes (word: this lane's bits, 0 for a lane
 // that takes no part), top-down, premultiplied.  Once the alpha is exactly 1
 // every later layer adds its colour times 0, so a lane stops there with the
-// same result.  The wave walks the group's shapes together, from the top of
-// `cand` (wave-uniform, a superset of every lane's bits): each shape is
-// composited by the lanes that hold it.  A lane meets its own shapes in its
-// own order, as a walk of its bits alone would, but the wave evaluates one
-// substance at a time, whose tag and record every lane reads alike.
+// same result.  The wave walks the shapes some lane holds together, from the
+// top: each shape is composited by the lanes that hold it.  A lane meets its
+// own shapes in its own order, as a walk of its bits alone would, but the
+// wave evaluates one substance at a time, whose tag and record every lane
+// reads alike.  Every lane of the wave calls it.
 __device__ __forceinline__ float4 group_composite(const SceneDesc &s, const TileTable *tt,
-                                                  uint32_t word, int n0, int ax, int ay, uint32_t cand)
+                                                  uint32_t word, int n0, int ax, int ay)
 {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    cand = __builtin_amdgcn_readfirstlane(cand);
+    uint32_t cand = wave_or(word);
     while (cand) {
         if (!__any(word != 0u)) break;
         const int b = 31 - __clz((int)cand);
@@ -943,38 +957,20 @@ __device__ __forceinline__ float4 group_composite(const SceneDesc &s, const Tile
     return acc;
 }
 
-// Accurate-mode colour of a grouped tile: over(group 3 .. group 0,
-// background), recomputing only the dirty groups' cached composites.  Groups
-// under an alpha of exactly 1 add nothing (their colour times 0): they are
-// neither read nor recomputed, and stay dirty.
-__device__ float4 grouped_color(const SceneDesc &s, TileTable *tt, Stack &st, int lane, int ax,
-                                int ay)
+// Accurate-mode colour of a grouped tile under the stack (s0, s1):
+// over(group 3 .. group 0, background).  Groups under an alpha of exactly 1
+// add nothing (their colour times 0) and are not walked.  Every lane of the
+// wave calls it, with valid false where it holds no section.
+__device__ __forceinline__ float4 grouped_color(const SceneDesc &s, const TileTable *tt, uint64_t s0, uint64_t s1,
+                                                bool valid, int ax, int ay)
 {
     const uint32_t q = __builtin_amdgcn_readfirstlane(tt->gq);
-    const uint32_t words[4] = {group_bits(st.s0, st.s1, 0u, q), group_bits(st.s0, st.s1, q, q),
-                               group_bits(st.s0, st.s1, 2u * q, q), group_bits(st.s0, st.s1, 3u * q, q)};
     float P0 = 0.f, P1 = 0.f, P2 = 0.f, A = 0.f;
-    uint32_t fresh = 0;
-    bool open = true;   // no group so far has brought the alpha to 1
-#pragma unroll
+#pragma unroll 1
     for (int g = 3; g >= 0; --g) {
-        open = open && A != 1.0f;
-        const bool stale = open && (st.dirty & (1u << g)) != 0u;
-        float4 gcol = make_float4(0.f, 0.f, 0.f, 0.f);
-        // every lane of the sweep step takes part in the walk (with no bits
-        // unless its group is stale)
-        if (__any(stale))
-            gcol = group_composite(s, tt, stale ? words[g] : 0u, (int)(g * q), ax, ay, tt->cand[g]);
-        if (stale) {
-            tt->gc[g][0][lane] = gcol.x;
-            tt->gc[g][1][lane] = gcol.y;
-            tt->gc[g][2][lane] = gcol.z;
-            tt->gc[g][3][lane] = gcol.w;
-            fresh |= 1u << g;
-        } else if (open) {
-            gcol = make_float4(tt->gc[g][0][lane], tt->gc[g][1][lane], tt->gc[g][2][lane],
-                               tt->gc[g][3][lane]);
-        }
+        const bool open = valid && A != 1.0f;
+        const uint32_t word = open ? group_bits(s0, s1, (uint32_t)g * q, q) : 0u;
+        const float4 gcol = group_composite(s, tt, word, (int)(g * q), ax, ay);
         if (open) {
             const float t = 1.0f - A;
             P0 = P0 + gcol.x * t;
@@ -983,7 +979,6 @@ __device__ float4 grouped_color(const SceneDesc &s, TileTable *tt, Stack &st, in
             A = A + gcol.w * t;
         }
     }
-    st.dirty &= ~fresh;
     {
         const float4 pm = make_float4(s.bg[0] * s.bg[3], s.bg[1] * s.bg[3], s.bg[2] * s.bg[3], s.bg[3]);
         const float t = 1.0f - A;
@@ -1134,119 +1129,214 @@ __device__ __forceinline__ uint32_t pixel_word(float4 c, bool rgba)
     return w;
 }
 
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ void write_pixel(const Frame &f, const SceneDesc &s, int x, int y, float4 color)
+{
+    const long long pix = (long long)y * s.width + x;
+    s.out[pix] = pixel_word(color, f.out_rgba != 0);
+    if (s.out_f32) s.out_f32[pix] = color;
+}
+
+// The colours of the `count` listed sections, a section a lane, whichever
+// lanes swept them; then every sweeping lane adds its sections' colour x area
+// in their order (head: its first), and the pixels that ended are written
+// (writePixelGlobal, Kernels.cl:1853-1862: the area-weighted mean).
+template <bool kCompact>
+__device__ __forceinline__ void color_sections(const Frame &f, const SceneDesc &s, const Column &c,
+                                               const int32_t *sidx, TileTable *tt, bool grouped, int lane, int count,
+                                               uint32_t head, float4 &acc, float &area_sum)
+{
+    SectionList &L = tt->sec;
+    wave_sync();
+    for (int e0 = 0; e0 < count; e0 += kWave) {
+        const int e = e0 + lane;
+        const bool valid = e < count;
+        const uint32_t info = valid ? L.info[e] : 0u;
+        const float4 bits = L.val[valid ? e : 0];
+        const int owner = (int)(info & 63u);
+        const int ax = __shfl(c.dx, owner), ay = __shfl(c.dy, owner) + (int)((info >> 6) & 0x1FFFu);
+        const uint64_t s0 = ((uint64_t)__float_as_uint(bits.y) << 32) | __float_as_uint(bits.x);
+        const uint64_t s1 = ((uint64_t)__float_as_uint(bits.w) << 32) | __float_as_uint(bits.z);
+        float4 col;
+        if (grouped) {
+            col = grouped_color(s, tt, s0, s1, valid, ax, ay);
+        } else {
+            bool positional = false;
+            if (valid)
+                col = determine_color<kCompact>(f, s, Stack{s0, s1}, sidx - lane + owner, tt, ax, ay, positional);
+        }
+        if (valid) {
+            const float adj = L.adj[e];
+            L.val[e] = make_float4(col.x * adj, col.y * adj, col.z * adj, col.w * adj);
+        }
+    }
+    wave_sync();
+    for (uint32_t e = head; e != kSecNone;) {
+        const float4 v = L.val[e];
+        const uint32_t info = L.info[e];
+        acc.x += v.x;
+        acc.y += v.y;
+        acc.z += v.z;
+        acc.w += v.w;
+        area_sum += L.adj[e];
+        if (info & kSecEnd) {
+            L.val[e] = acc;
+            L.adj[e] = area_sum;
+            acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            area_sum = 0.0f;
+        }
+        e = info >> 24;
+    }
+    wave_sync();
+    for (int e0 = 0; e0 < count; e0 += kWave) {
+        const int e = e0 + lane;
+        const uint32_t info = e < count ? L.info[e] : 0u;
+        const int owner = (int)(info & 63u);
+        const int ax = __shfl(c.dx, owner), ay = __shfl(c.dy, owner) + (int)((info >> 6) & 0x1FFFu);
+        if (info & kSecEnd) {
+            const float4 a = L.val[e];
+            const float w = L.adj[e];
+            write_pixel(f, s, ax, ay, make_float4(a.x / w, a.y / w, a.z / w, a.w / w));
+        }
+    }
+    wave_sync();
+}
+
 // renderThresholdArray + calculatePixel + horizontalAdvance + sectionColor
 // (Kernels.cl:1724-1742, 1826-1851, 1881-1916, 1978-2028).  The reference
 // loops over a column's pixels and, inside, over each pixel's sections; here
-// one loop steps either a section or the end of a pixel.  The sections and
-// their arithmetic are the same, but lanes of a wave whose pixels hold
-// different numbers of sections no longer wait for each other at every
-// pixel, only at the end of their columns (the 4096^2 frame: 57.4 -> 51.9 ms).
+// one loop steps a section of every lane that has one left, whatever its
+// pixel, so lanes only wait for each other at the end of their columns (the
+// 4096^2 frame: 57.4 -> 51.9 ms).
+// The loop only sweeps: it appends each section, its area and the stack it
+// lies under to a list in LDS, and when 192 are listed the whole wave gives
+// them their colours, a section a lane (color_sections).  A step of the sweep
+// has ~21 of 64 lanes in a section; colouring them there kept the colour
+// walks, half of the frame's vector instructions, at that occupancy, and a
+// lone busy column waited for each of its colours.  Now the 4096^2 frame
+// takes 35.2 ms against 43.5 (1.34e10 vector instructions against 1.75e10)
+// and an 800x600 frame of 256-px tiles, 250 waves in all, 27 against 45.  A
+// list of 192 keeps five blocks in a CU's LDS: 171 entries take 35.6 ms.
+// Every lane of the wave calls it; ok: the lane has a column to sweep.
 template <bool kCompact>
 __device__ uint32_t render(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, Stack st,
-                           int32_t *sidx, TileTable *tt, bool nz)
+                           int32_t *sidx, TileTable *tt, bool nz, bool ok)
 {
     int32_t *const wind = sidx + kWindOffset * kWave;
+    SectionList &L = tt->sec;
     Sweep p;
     p.current = 0; p.num_active = 0;
     p.sx0 = 0.0f; p.sy0 = 0.0f; p.sx1 = 1.0f; p.sy1 = 0.0f;
     const bool stochastic = f.stochastic != 0.0f;
-    if (stochastic) {   // initRandomField (Kernels.cl:1597-1606)
+    p.rnd = 0;
+    if (stochastic && ok) {   // initRandomField (Kernels.cl:1597-1606)
         const uint32_t start = c.unique & (uint32_t)f.random_mask;
         p.rnd = __float_as_uint(f.random[start]) & (uint32_t)f.random_mask;
-    } else {
-        p.rnd = 0;
     }
-    long guard = kSectionGuard;
-    int ay = c.dy;
-    int yint = 0;
-    const bool grouped = kCompact && tt->grouped;
+    uint32_t status = 0;
+    int guard = (int)kSectionGuard;
+    uint32_t row = 0;
     const int lane = threadIdx.x & (kWave - 1);
-    st.dirty = 0xFu;
-    if (grouped) st.gm = __builtin_amdgcn_readfirstlane(tt->gm);
-    const uint32_t gq = grouped ? __builtin_amdgcn_readfirstlane(tt->gq) : 32u;
+    const bool grouped = kCompact && __builtin_amdgcn_readfirstlane((uint32_t)tt->grouped) != 0u;
     p.pixel_y = 1.0f;
-    if (!(p.pixel_y <= c.float_height)) return 0;
+    bool alive = ok && p.pixel_y <= c.float_height;
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float area_sum = 0.0f;
-    if (grouped) {
-        // picture colours depend on the pixel: their groups are stale
-        const uint64_t p0 = st.s0 & tt->pic0, p1 = st.s1 & tt->pic1;
-        st.dirty |= (group_bits(p0, p1, 0u, gq) ? 1u : 0u) | (group_bits(p0, p1, gq, gq) ? 2u : 0u) |
-                    (group_bits(p0, p1, 2u * gq, gq) ? 4u : 0u) | (group_bits(p0, p1, 3u * gq, gq) ? 8u : 0u);
-    }
+    int count = 0;                              // listed sections (wave-uniform)
+    uint32_t head = kSecNone, last = kSecNone;  // this lane's first and last
     for (;;) {
-        if ((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y)) {
-            if (--guard < 0) return kStatusGuard;
-            vertical_advance(q, c, p, st, wind, nz);
-            if (q.spilled || q.overflow) return 0;
-            // horizontalAdvance with thresholdMidXLow (Kernels.cl:916-926)
-            float nx;
-            if (p.current < p.num_active) {
-                const Thr t = q.get(p.current);
-                const uint32_t h = q.get_h(p.current);
-                float x;
-                if (f.coverage_mode == GUDNI_COVERAGE_REFERENCE) {
-                    const float ymid = p.sy0 + ((p.sy1 - p.sy0) * 0.5f);
-                    x = intersect_x(h, t, ymid);
-                } else if (t.left == t.right) {
-                    x = t.left;
+        const bool running = __any(alive);
+        bool have = false, end = false;
+        float adj = 0.0f;
+        uint64_t s0 = 0, s1 = 0;
+        const uint32_t at_row = row;
+        if (alive) {
+            bool done = !((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y));
+            if (done) {
+                // a pixel without sections (its records hold NaN): 0 / 0
+                const float nan = __int_as_float(0x7FC00000);
+                write_pixel(f, s, c.dx, c.dy + (int)row, make_float4(nan, nan, nan, nan));
+            } else if (--guard < 0) {
+                status = kStatusGuard;
+                alive = false;
+            } else {
+                vertical_advance(q, c, p, st, wind, nz);
+                if (q.spilled || q.overflow) {
+                    alive = false;
                 } else {
-                    // the same mid point, relative to the threshold's start
-                    const float sy = hdr_pos(h) ? t.top : t.bottom;
-                    const float d = (p.sy0 - sy) + ((p.sy1 - p.sy0) * 0.5f);
-                    x = (d * inv_slope(h, t)) + t.left;
+                    // horizontalAdvance with thresholdMidXLow (Kernels.cl:916-926)
+                    float nx = 1.0f;
+                    uint32_t h = 0;
+                    const bool crossing = p.current < p.num_active;
+                    if (crossing) {
+                        const Thr t = q.get(p.current);
+                        h = q.get_h(p.current);
+                        float x;
+                        if (f.coverage_mode == GUDNI_COVERAGE_REFERENCE) {
+                            const float ymid = p.sy0 + ((p.sy1 - p.sy0) * 0.5f);
+                            x = intersect_x(h, t, ymid);
+                        } else if (t.left == t.right) {
+                            x = t.left;
+                        } else {
+                            // the same mid point, relative to the threshold's start
+                            const float sy = hdr_pos(h) ? t.top : t.bottom;
+                            const float d = (p.sy0 - sy) + ((p.sy1 - p.sy0) * 0.5f);
+                            x = (d * inv_slope(h, t)) + t.left;
+                        }
+                        nx = (x >= 1.0f) ? 0.0f : cl_max(0.0f, x);
+                    }
+                    p.sx0 = p.sx1;
+                    p.sx1 = nx;
+                    const float area = (p.sx1 - p.sx0) * (p.sy1 - p.sy0);
+                    adj = area;
+                    if (stochastic) {   // getRandom (Kernels.cl:1608-1613)
+                        p.rnd = (p.rnd + 1u) & (uint32_t)f.random_mask;
+                        adj = area + (area * f.random[p.rnd] * f.stochastic);
+                    }
+                    have = true;
+                    s0 = st.s0;
+                    s1 = st.s1;
+                    if (crossing) st.cross<kCrossRight>(h, wind, nz);
+                    ++p.current;
+                    done = end = !((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y));
                 }
-                nx = (x >= 1.0f) ? 0.0f : cl_max(0.0f, x);
-            } else {
-                nx = 1.0f;
             }
-            p.sx0 = p.sx1;
-            p.sx1 = nx;
-            float4 col;
-            if (grouped) {
-                col = grouped_color(s, tt, st, lane, c.dx, ay);
-            } else {
-                bool positional = false;
-                col = determine_color<kCompact>(f, s, st, sidx, tt, c.dx, ay, positional);
-            }
-            const float area = (p.sx1 - p.sx0) * (p.sy1 - p.sy0);
-            float adj = area;
-            if (stochastic) {   // getRandom (Kernels.cl:1608-1613)
-                p.rnd = (p.rnd + 1u) & (uint32_t)f.random_mask;
-                adj = area + (area * f.random[p.rnd] * f.stochastic);
-            }
-            acc.x += col.x * adj;
-            acc.y += col.y * adj;
-            acc.z += col.z * adj;
-            acc.w += col.w * adj;
-            area_sum += adj;
-            if (p.current < p.num_active) st.cross<kCrossRight>(q.get_h(p.current), wind, nz);
-            ++p.current;
-        } else {
-            // the pixel's last section is done: its colour is the area-weighted
-            // mean (writePixelGlobal, Kernels.cl:1853-1862), then the next pixel
-            const float4 color = make_float4(acc.x / area_sum, acc.y / area_sum, acc.z / area_sum,
-                                             acc.w / area_sum);
-            const long long pix = (long long)(c.dy + yint) * s.width + c.dx;
-            s.out[pix] = pixel_word(color, f.out_rgba != 0);
-            if (s.out_f32) s.out_f32[pix] = color;
-            p.sx0 = 0.0f;
-            p.sy0 = p.pixel_y;
-            ++ay;
-            ++yint;
-            p.pixel_y += 1.0f;
-            if (!(p.pixel_y <= c.float_height)) break;
-            acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            area_sum = 0.0f;
-            if (grouped) {
-                const uint64_t p0 = st.s0 & tt->pic0, p1 = st.s1 & tt->pic1;
-                st.dirty |= (group_bits(p0, p1, 0u, gq) ? 1u : 0u) | (group_bits(p0, p1, gq, gq) ? 2u : 0u) |
-                            (group_bits(p0, p1, 2u * gq, gq) ? 4u : 0u) |
-                            (group_bits(p0, p1, 3u * gq, gq) ? 8u : 0u);
+            if (done) {   // the next pixel
+                p.sx0 = 0.0f;
+                p.sy0 = p.pixel_y;
+                ++row;
+                p.pixel_y += 1.0f;
+                alive = p.pixel_y <= c.float_height;
             }
         }
+        const uint64_t mask = __ballot(have);
+        const int n = __popcll(mask);
+        if (count + n > kSections || !running) {
+            color_sections<kCompact>(f, s, c, sidx, tt, grouped, lane, count, head, acc, area_sum);
+            count = 0;
+            head = last = kSecNone;
+            if (!running) break;
+        }
+        if (have) {
+            const uint32_t e = (uint32_t)count + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+            L.val[e] = make_float4(__uint_as_float((uint32_t)s0), __uint_as_float((uint32_t)(s0 >> 32)),
+                                   __uint_as_float((uint32_t)s1), __uint_as_float((uint32_t)(s1 >> 32)));
+            L.adj[e] = adj;
+            L.info[e] = (uint32_t)lane | (at_row << 6) | (end ? kSecEnd : 0u) | (kSecNone << 24);
+            if (last == kSecNone) head = e;
+            else reinterpret_cast<uint8_t *>(&L.info[last])[3] = (uint8_t)e;
+            last = e;
+        }
+        count += n;
     }
-    return 0;
+    return status;
 }
 
 // initTileState / isActiveThread (Kernels.cl:1692-1722)
@@ -1331,9 +1421,7 @@ __device__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t 
             tt->color[n] = col;
             all_add = all_add && (tag & kTagCompoundMask) == kTagAdd;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
         // grouped colours need every shape added with its own substance
         bool distinct = true;
         for (int n = lane; n < c.num_shapes; n += kWave) {
@@ -1356,7 +1444,6 @@ __device__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t 
             tt->grouped = grouped_tile ? 1 : 0;
             const uint32_t gq = c.num_shapes > 4 ? (uint32_t)(c.num_shapes + 3) / 4u : 1u;
             tt->gq = gq;
-            tt->gm = (65536u + gq - 1u) / gq;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -1372,26 +1459,10 @@ __device__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t 
         generate<kCompact>(f, s, q, c, active, lane, (float)x0 - 1.0f, (float)x1 + 1.0f, sidx, bits,
                            s0, s1, c0, c1, any_nonzero);
     }
-    if (kCompact) {
-        // a lane's stack only ever holds bits of shapes it took a record or
-        // an enclosure of: their union over the wave bounds the colour walks
-        uint64_t u0 = c0, u1 = c1;
-        for (int o = 32; o > 0; o >>= 1) {
-            u0 |= __shfl_xor(u0, o);
-            u1 |= __shfl_xor(u1, o);
-        }
-        if (lane == 0) {
-            const uint32_t q = tt->gq;
-            for (uint32_t g = 0; g < 4u; ++g) tt->cand[g] = group_bits(u0, u1, g * q, q);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
     const bool ok = active && !q.spilled && !q.overflow;
     const long long t1 = timed ? clock64() : 0;
     if (ok && f.dump_qlen) dump_queue<kCompact>(f, q, dslot, true, c0, c1);
-    if (ok) radix_sort_queue(q, reinterpret_cast<uint16_t *>(&tt->gc[0][0][0]) + lane, s.sort_bits,
+    if (ok) radix_sort_queue(q, reinterpret_cast<uint16_t *>(&tt->sec) + lane, s.sort_bits,
                              c.float_height);
     if (ok && f.dump_qlen) {
         dump_queue<kCompact>(f, q, dslot, false, c0, c1);
@@ -1424,7 +1495,7 @@ __device__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t 
     }
     const long long t2 = timed ? clock64() : 0;
     // only a lane that walked a nonzero-fill shape keeps winding counters
-    if (ok) status = render<kCompact>(f, s, q, c, Stack{s0, s1, 0u}, sidx, tt, any_nonzero);
+    status = render<kCompact>(f, s, q, c, Stack{s0, s1}, sidx, tt, any_nonzero, ok);
     if (active && q.overflow) status |= kStatusOverflow;
     if (!active && f.dump_qlen) f.dump_qlen[dslot] = -1;
     if (timed) {

@@ -1,0 +1,40 @@
+"""The sweep's section list: frames whose pixels hold fewer, exactly as many
+and more sections than a list (192) equal the oracle's bit for bit, in one
+column and in several, with colours grouped and walked."""
+import numpy as np
+import pytest
+
+import gudni_amd as G
+from gudni_amd import scenes as S
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def teeth(n, width, height):
+    """One shape of n upright bars inside every pixel column, alternating
+    between two colours' shapes: 2 n + 1 sections in every pixel."""
+    bars = [[], []]
+    for x in range(width):
+        for i in range(n):
+            x0 = x + (4 * i + 1) / (4.0 * n + 2)
+            bars[i % 2].append(S.rectangle_pairs(x0, -1.0, x0 + 1.5 / (4.0 * n + 2), height + 1.0))
+    shapes = [(S.solid_tag(i), b) for i, b in enumerate(bars) if b]
+    return S.build_scene(width, height, shapes, [[0.9, 0.2, 0.1, 0.6], [0.1, 0.4, 0.8, 0.7]], name=f"teeth{n}")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,width,height", [(1, 1, 1), (95, 1, 3), (96, 1, 2), (31, 2, 2), (48, 2, 3), (97, 3, 2),
+                                            (200, 1, 2), (1, 70, 9), (2, 64, 64)])
+def test_section_lists(n, width, height, mode):
+    scene = teeth(n, width, height)
+    spec = G.default_spec(coverage_mode=mode)
+    want = H.oracle_render(scene, spec)
+    assert want["rc"] == 0
+    r = G.Rasterizer(spec)
+    try:
+        got, f32 = H.gpu_render_level2(r, scene, spec)
+    finally:
+        r.close()
+    assert np.array_equal(got, want["out"]), H.first_mismatch(got, want["out"])
+    assert np.array_equal(f32, want["f32"])
