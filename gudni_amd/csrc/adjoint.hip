@@ -933,7 +933,7 @@ __device__ __forceinline__ void adj_unit(const Frame &f, const AdjDesc &d, int l
     // optional phase clocks (wave-uniform points): [0] A generate [1] A sort
     // [2] A sweep [3] B generate [4] B sort [5] B sweep [6] C [7] units
     unsigned long long *clk = f.stage_cycles;
-    uint16_t *hist = reinterpret_cast<uint16_t *>(&tt->sec) + lane;   // sort histogram
+    uint16_t *hist = tt->hist + lane;   // sort histogram
     long long tclk = clk ? clock64() : 0;
     auto stamp = [&](int i) {
         if (!clk) return;

@@ -63,6 +63,7 @@ constexpr int kFastCapLog2 = 7;           // 128-record rings in the fast pass
 constexpr long kSectionGuard = 1L << 22;  // sweep-length bound per column: the
                                           // longest legitimate sweep is 256 rows
                                           // x (2*4096+1) sections = 2.1M
+constexpr int kRadixMaxBits = 5;          // widest digit of the sort's radix pass
 constexpr int kMaxBisect = 64;            // bifurcation bound per intersection
 
 // status codes a lane can raise (bit flags in the launch's status word)
@@ -392,9 +393,140 @@ __device__ __forceinline__ void search_pair(Trav &l, Trav &r, const GUDNI_CONST 
     }
 }
 
-// buildThresholdArray (Kernels.cl:1540-1595).  The shape and strand loops
-// are wave-uniform (every lane walks the tile's whole shape list); only the
-// range test, tree searches and record pushes diverge.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A wave's list of sections waiting for their colours: per section its area
+// (adj) and the stack it lies under, which the colour pass replaces by colour
+// x area.  info: the lane that swept it (bits 0..5), its pixel's row in that
+// lane's segment (6..18), whether it is its pixel's last (kSecEnd), and the
+// lane's next section in the list (24..31, kSecNone: none).
+constexpr int kSections = 192;             // three full waves of colours
+constexpr uint32_t kSecEnd = 1u << 19, kSecNone = 0xFFu;
+struct SectionList {
+    float4 val[kSections];
+    float adj[kSections];
+    uint32_t info[kSections];
+};
+
+// A wave's list of strands that generation walks: extents (left x, right x,
+// top, bottom) and the strand's place in the heap (16-byte units) and meta
+// word (size in 8-byte units, the shape's index in its group of 64 << 16,
+// kStrandNonzero, kStrandReversed, kStrandFar: not to be judged by extents).
+constexpr int kStrands = 192;
+constexpr uint32_t kStrandNonzero = 1u << 22, kStrandReversed = 1u << 23, kStrandFar = 1u << 24;
+struct StrandList {
+    float4 box[kStrands];
+    uint2 ref[kStrands];
+};
+
+// Per-wave LDS table of a compact tile's shapes by tile-local index: tag,
+// and the solid colour (in the coverage mode's form) or, for a picture or
+// gradient, the substance record itself.
+struct TileTable {
+    uint64_t tag[128];
+    float4 color[128];
+    union {
+        SectionList sec;       // the sweep's sections
+        StrandList strands;    // generation's strands
+        uint16_t hist[(1 << kRadixMaxBits) * kWave];   // the sort's histogram
+    };
+    uint64_t pic0, pic1;   // tile-local shapes whose substance is a picture
+    int grouped;           // the tile qualifies for grouped colours
+    // colour group g holds tile-local shapes [g gq, (g+1) gq), gq = ceil(n / 4)
+    // for a tile of n shapes
+    uint32_t gq;
+};
+// traverseTree (Kernels.cl:1378-1408)'s column-relative view of a strand.
+__device__ __forceinline__ Trav strand_view(const GUDNI_CONST uint8_t *strand, float dx, float dy)
+{
+    const float2 right = ld2(strand + 8);
+    const float4 lc = ld4(strand + 16);
+    Trav t;
+    t.right = make_float2(right.x - dx, right.y - dy);
+    t.left = make_float2(lc.x - dx, lc.y - dy);
+    t.ctl = make_float2(lc.z - dx, lc.w - dy);
+    t.xpos = 0.0f;
+    t.index = 0;
+    return t;
+}
+
+// Bounds (lo, hi) on the y of an x-monotone curve over [x0, x1]: the hull of
+// the piece between the parameters of x0 and x1 (the roots of its x
+// polynomial, by hardware reciprocal and square root: what is off is covered
+// by the caller's margin).  False where the parameters are not well defined.
+__device__ __forceinline__ bool curve_bounds(const Trav &t, float x0, float x1, float &lo, float &hi)
+{
+    const float a = (t.left.x - t.ctl.x) + (t.right.x - t.ctl.x), b = t.ctl.x - t.left.x;
+    const float b2 = b * b;
+    const float d0 = b + __builtin_amdgcn_sqrtf(fmaxf(b2 - a * (t.left.x - x0), 0.0f));
+    const float d1 = b + __builtin_amdgcn_sqrtf(fmaxf(b2 - a * (t.left.x - x1), 0.0f));
+    const float t0 = fminf(fmaxf((x0 - t.left.x) * __builtin_amdgcn_rcpf(d0), 0.0f), 1.0f);
+    const float t1 = fminf(fmaxf((x1 - t.left.x) * __builtin_amdgcn_rcpf(d1), 0.0f), 1.0f);
+    // blossom of the y polynomial: (t0,t0), (t0,t1), (t1,t1)
+    const float u0 = t.left.y + (t.ctl.y - t.left.y) * t0, v0 = t.ctl.y + (t.right.y - t.ctl.y) * t0;
+    const float u1 = t.left.y + (t.ctl.y - t.left.y) * t1, v1 = t.ctl.y + (t.right.y - t.ctl.y) * t1;
+    const float ya = u0 + (v0 - u0) * t0, yb = u0 + (v0 - u0) * t1, yc = u1 + (v1 - u1) * t1;
+    lo = fminf(lo, fminf(ya, fminf(yb, yc)));
+    hi = fmaxf(hi, fmaxf(ya, fmaxf(yb, yc)));
+    return d0 > 1e-3f && d1 > 1e-3f;
+}
+
+// Whether a strand that covers the column passes wholly above its segment
+// (-1), wholly below (1) or may meet it (0).  spawn's lines run between points
+// of the curve under the left border, of the one under the right border, and
+// from one curve to the other.  A border's y is a chord's, and a flat chord
+// lies within 0.25 (in x plus y) of its curve; so all of them lie outside the
+// segment where both curves do, over the column widened by half a pixel, by
+// the margin: 2 pixels and 1/256 of the curves' extent.
+__device__ __forceinline__ int strand_side(const SceneDesc &s, uint2 ref, float dx, float dy, float height)
+{
+    if (ref.y & kStrandFar) return 0;
+    const GUDNI_CONST uint8_t *strand = ro(s.geo) + 16ull * ref.x;
+    Trav l = strand_view(strand, dx, dy), r = l;
+    l.xpos = cl_max(0.0f, l.left.x);
+    r.xpos = cl_min(1.0f, l.right.x);
+    search_pair(l, r, strand + 32, ((int)(ref.y & 0xFFFFu) - 4) / 2, dx, dy);
+    float lo = FLT_MAX, hi = -FLT_MAX;
+    bool known = curve_bounds(l, fmaxf(l.left.x, -0.5f), fminf(1.5f, l.right.x), lo, hi);
+    float extent = (l.right.x - l.left.x) + fabsf(l.ctl.y - l.left.y) + fabsf(l.right.y - l.ctl.y);
+    if (l.index != r.index) {
+        known = curve_bounds(r, fmaxf(r.left.x, -0.5f), fminf(1.5f, r.right.x), lo, hi) && known;
+        extent = fmaxf(extent, (r.right.x - r.left.x) + fabsf(r.ctl.y - r.left.y) + fabsf(r.right.y - r.ctl.y));
+    }
+    if (!known) return 0;
+    const float margin = 2.0f + extent * (1.0f / 256.0f);
+    return hi <= -margin ? -1 : (lo >= height + margin ? 1 : 0);
+}
+
+// buildThresholdArray (Kernels.cl:1540-1595): every column of the wave takes
+// the strands of its tile's shapes in order and emits their thresholds.
+//
+// The walk is a lane's own.  Per group of 64 shapes the wave lists the
+// strands of those that reach its columns, with their extents; each lane then
+// marks the strands that cross its own segment and runs only those, one a
+// step, so a step serves a different strand in every lane and there are as
+// many steps as the busiest lane has crossing strands (walking strand by
+// strand, the wave ran every strand that crossed any of its 64 columns).
+// What the other strands do to a column follows from their extents:
+//  * left of or right of the column (the reference's own range test): nothing;
+//  * wholly below the segment, by a pixel or more: no threshold, and none that
+//    starts at or above its top;
+//  * wholly above it, by a pixel or more: no threshold either, but a strand
+//    that covers the column's left border has a persistent threshold there,
+//    which ends above the top: the segment's enclosure flips (checkInRange
+//    holds and xpos is 0, so the first line starts on the border).
+// A strand with a coordinate at or beyond 2^20 (whose rounding the pixel does
+// not cover) or NaN is always run.  The strands whose extents do not settle it
+// are then bounded within the very column (strand_side): on the 4096^2 frame
+// a wave lists 510 strands, 200 reach some of its columns, 57 of them a
+// lane's segment by their extents, and a column takes 5.5 records.
+// Generation took 95e9 wave cycles of that frame and takes 67e9 (35.2 -> 33.6
+// ms); 512^2 scribbles 51e9 -> 31e9 (20.8 -> 17.9 ms).
 //
 // kCompact (a tile of at most maxShapes shapes, i.e. every tile above the
 // 8-pixel floor): the 127-shape cap cannot bind, and the column's shape bit
@@ -405,105 +537,225 @@ __device__ __forceinline__ void search_pair(Trav &l, Trav &r, const GUDNI_CONST 
 // instead of chasing shapeIndices[b] -> shape record -> substance in memory.
 // `contrib` records which n contributed, so the reference's labels can be
 // recovered (dump path).
-template <bool kCompact>
-__device__ void generate(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, bool active, int lane,
-                         float span0, float span1, int32_t *sidx,
-                         uint32_t &shape_bits, uint64_t &stack0, uint64_t &stack1,
-                         uint64_t &contrib0, uint64_t &contrib1, bool &any_nonzero)
+// emit(place, meta, label and rule bits, added, enclosed) runs one strand.
+template <bool kCompact, class Emit>
+__device__ __forceinline__ void walk_strands(const Frame &f, const SceneDesc &s, const Queue &q, const Column &c,
+                                             bool active, int lane, float span0, float span1, int32_t *sidx,
+                                             StrandList &list, uint32_t &shape_bits, uint64_t &stack0,
+                                             uint64_t &stack1, uint64_t &contrib0, uint64_t &contrib1,
+                                             bool &any_nonzero, Emit &&emit)
 {
     const float dx = (float)c.dx, dy = (float)c.dy;
     const uint32_t max_shapes = (uint32_t)f.max_shapes;
-    // The shape and strand walks are the same for every lane of the wave;
-    // readfirstlane makes that explicit so their loads go to the scalar unit.
     const int num_shapes = (int)__builtin_amdgcn_readfirstlane(c.num_shapes);
     const int shape_start = (int)__builtin_amdgcn_readfirstlane(c.shape_start);
-    // A shape none of whose strands reaches a column adds no threshold and no
-    // enclosure there, so it gets no shape bit and can be skipped.  The wave
-    // tests 64 shapes at a time against [span0, span1] (its columns' x extent
-    // widened by a pixel, a superset of checkInRange's per-column test) and
-    // walks only the candidates, in shape order.
-    // A lane also skips a shape lying wholly below its segment (every point
-    // at least a pixel under the segment's bottom): its thresholds all start
-    // at or below RENDEREND, so none is added and none encloses.
-    const float below = dy + c.float_height + 1.0f;
+    const float below = dy + c.float_height + 1.0f, above = dy - 1.0f;
+    float lowest = active ? below : -FLT_MAX;   // nothing below it reaches the wave
+    for (int o = 32; o > 0; o >>= 1) lowest = fmaxf(lowest, __shfl_xor(lowest, o));
     bool alive = active;
     for (int base = 0; base < num_shapes; base += kWave) {
         alive = alive && shape_bits < max_shapes && !q.spilled && !q.overflow;
         if (!__any(alive)) break;
+        // a shape none of whose strands reaches a column adds no threshold
+        // and no enclosure there: those that miss [span0, span1] (the wave's
+        // columns widened by a pixel) are left out
         const int ni = base + lane;
-        bool cand = false;
-        float ymin = 0.0f;
+        uint32_t ns = 0, place = 0, rule = 0;
+        float shape_top = 0.0f;
         if (ni < num_shapes) {
             const float4 b = s.bounds[shape_start + ni];
-            cand = (b.x <= span1) && (b.z > span0);
-            ymin = b.y;
-        }
-        uint64_t pending = __ballot(cand);
-        while (pending) {
-            const int i = __ffsll((long long)pending) - 1;
-            const int n = base + i;
-            pending &= pending - 1;
-            const float shape_top = __shfl(ymin, i);
-            alive = alive && shape_bits < max_shapes && !q.spilled && !q.overflow;
-            if (!alive || shape_top >= below) continue;
-        const int shape_index = shape_start + n;
-        const GUDNI_CONST uint32_t *srec =
-            reinterpret_cast<const GUDNI_CONST uint32_t *>(ro(s.shapes) + shape_index);
-        uint64_t offset = 16ull * __builtin_amdgcn_readfirstlane(srec[2]);
-        const uint32_t num_strands = __builtin_amdgcn_readfirstlane(srec[3]);
-        const bool nonzero = (__builtin_amdgcn_readfirstlane(srec[1]) & (uint32_t)(kTagNonzero >> 32)) != 0u;
-        any_nonzero = any_nonzero || nonzero;   // this lane walked a nonzero-fill shape
-        const uint32_t label = kCompact ? (uint32_t)n : shape_bits;
-        bool added = false, enclosed_shape = false;
-        int32_t w0 = 0;   // winding number of the segment's top-left corner (nonzero fill)
-        for (uint32_t si = 0; si < num_strands; ++si) {
-            const GUDNI_CONST uint8_t *strand = ro(s.geo) + offset;
-            // u16 size in 8-byte units, then u16 flags: read as one dword
-            const uint32_t head = *reinterpret_cast<const GUDNI_CONST uint32_t *>(strand);
-            const uint32_t size = head & 0xFFFFu;
-            const bool reversed = nonzero && ((head >> 16) & GUDNI_STRAND_REVERSED) != 0u;
-            const uint32_t rule = nonzero ? (kNonzero | (reversed ? kReversed : 0u)) : 0u;
-            bool enclosed_strand = false;
-            // traverseTree (Kernels.cl:1378-1408)
-            const float2 right = ld2(strand + 8);
-            const float4 lc = ld4(strand + 16);
-            Trav l;
-            l.right = make_float2(right.x - dx, right.y - dy);
-            l.left = make_float2(lc.x - dx, lc.y - dy);
-            l.ctl = make_float2(lc.z - dx, lc.w - dy);
-            l.xpos = 0.0f;
-            l.index = 0;
-            if (l.left.x <= 1.0f && l.right.x > 0.0f) {
-                Trav r = l;
-                l.xpos = cl_max(0.0f, l.left.x);
-                r.xpos = cl_min(1.0f, l.right.x);
-                const int tree_size = ((int)size - 4) / 2;
-                search_pair(l, r, strand + 32, tree_size, dx, dy);
-                spawn(q, c, label | rule, l, r, added, enclosed_strand);
+            shape_top = b.y;
+            if (b.x <= span1 && b.z > span0 && !(b.y >= lowest)) {
+                const ShapeRec r = s.shapes[shape_start + ni];
+                ns = r.num_strands;
+                place = r.geo_start;
+                rule = (r.tag & kTagNonzero) ? kStrandNonzero : 0u;
             }
-            offset += 8u * size;
-            enclosed_shape = enclosed_shape != enclosed_strand;
-            // a strand crossing the left border above the segment adds the
-            // sign of its original x direction (coming down that border)
-            if (enclosed_strand) w0 += reversed ? -1 : 1;
         }
-        if (nonzero) enclosed_shape = w0 != 0;
-        if (enclosed_shape) {
-            if (label < 64u) stack0 ^= 1ull << label;
-            else stack1 ^= 1ull << (label - 64u);
+        uint32_t start = ns;
+        for (int o = 1; o < kWave; o <<= 1) {
+            const uint32_t t = __shfl_up(start, (unsigned)o);
+            if (lane >= o) start += t;
         }
-        if (added || enclosed_shape) {
-            if (nonzero) sidx[(kWindOffset + (int)label) * kWave] = w0;
-            if (kCompact) {
-                if (label < 64u) contrib0 |= 1ull << label;
-                else contrib1 |= 1ull << (label - 64u);
-            } else if (shape_bits < max_shapes) {
-                sidx[(int)shape_bits * kWave] = shape_index;
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)start, kWave - 1);
+        start -= ns;
+        uint64_t enc = 0, add = 0;   // shapes of the group that enclose the corner; that added records
+        int cur = -1;                // the nonzero-fill shape whose winding number w is being summed
+        int32_t w = 0;
+        auto label_of = [&](int k) -> uint32_t {
+            return kCompact ? (uint32_t)(base + k)
+                            : shape_bits + (uint32_t)__popcll((enc | add) & ((1ull << k) - 1ull));
+        };
+        auto close_winding = [&]() {
+            if (cur < 0) return;
+            if (w != 0) enc |= 1ull << cur;
+            const uint32_t label = label_of(cur);
+            if ((((enc | add) >> cur) & 1ull) && label < max_shapes) sidx[(kWindOffset + (int)label) * kWave] = w;
+            cur = -1;
+        };
+        uint32_t listed = 0;         // strands of this lane's shape listed so far
+        uint32_t n = 0;              // strands in the list
+        for (uint32_t w0 = 0; w0 < total;) {
+            const uint32_t w1 = min(total, w0 + (uint32_t)kStrands - n);
+            wave_sync();
+            while (listed < ns && start + listed < w1) {
+                const GUDNI_CONST uint8_t *p = ro(s.geo) + 16ull * place;
+                const float4 h = ld4(p), first = ld4(p + 16);
+                const uint32_t head = __float_as_uint(h.x), size = head & 0xFFFFu;
+                float lo = h.w, hi = h.w, far = fmaxf(fabsf(h.z), fabsf(h.w));
+                bool nan = !(h.z == h.z) || !(h.w == h.w);
+                const int m = (int)size / 2;   // float4s of the strand
+                float4 v = first;
+                for (int i = 1;;) {
+                    lo = fminf(lo, fminf(v.y, v.w));
+                    hi = fmaxf(hi, fmaxf(v.y, v.w));
+                    far = fmaxf(far, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+                    nan = nan || !(v.x == v.x) || !(v.y == v.y) || !(v.z == v.z) || !(v.w == v.w);
+                    if (++i >= m) break;
+                    v = ld4(p + 16 * i);
+                }
+                const bool wild = nan || far >= 1048576.0f;
+                if (wild) {
+                    lo = shape_top;
+                    hi = INFINITY;
+                }
+                const uint32_t e = n + start + listed - w0;
+                list.box[e] = make_float4(first.x, h.z, lo, hi);
+                list.ref[e] = make_uint2(place, size | ((uint32_t)lane << 16) | rule | (wild ? kStrandFar : 0u) |
+                                                    (rule && ((head >> 16) & GUDNI_STRAND_REVERSED) ? kStrandReversed : 0u));
+                place += size / 2;
+                ++listed;
             }
-            shape_bits += 1u;
+            wave_sync();
+            // of these, the list keeps those that reach the wave's columns
+            const uint32_t end = n + (w1 - w0);
+            for (uint32_t e0 = n; e0 < end; e0 += kWave) {
+                const uint32_t e = e0 + (uint32_t)lane;
+                float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+                uint2 ref = make_uint2(0u, 0u);
+                if (e < end) {
+                    b = list.box[e];
+                    ref = list.ref[e];
+                }
+                const bool keep = e < end && b.x <= span1 && b.y > span0 && !(b.z >= lowest);
+                const uint64_t mask = __ballot(keep);
+                if (keep) {
+                    const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                    list.box[at] = b;
+                    list.ref[at] = ref;
+                }
+                n += (uint32_t)__popcll(mask);
+            }
+            w0 = w1;
+            if (w0 < total && n <= (uint32_t)kStrands / 2) continue;   // room for more
+            wave_sync();
+            uint32_t todo[kStrands / 32];   // strands that this lane runs
+#pragma unroll
+            for (int g = 0; g < kStrands / 32; ++g) {
+                uint32_t m = 0;
+                const int e0 = 32 * g, e1 = min(e0 + 32, (int)n);
+                for (int e = e0; e < e1; ++e) {
+                    const float4 b = list.box[e];
+                    const uint32_t meta = __builtin_amdgcn_readfirstlane(list.ref[e].y);
+                    const float lx = b.x - dx;
+                    const bool in = lx <= 1.0f && b.y - dx > 0.0f;
+                    const bool over = b.w <= above && !(meta & kStrandNonzero);
+                    if (in && !over && !(b.z >= below)) m |= 1u << (e - e0);
+                    if (in && over && lx <= 0.0f) enc ^= 1ull << ((meta >> 16) & 63u);
+                }
+                todo[g] = alive ? m : 0u;
+            }
+            // of those, the ones whose curves come near the segment in this
+            // very column
+#pragma unroll
+            for (int g = 0; g < kStrands / 32; ++g) {
+                uint32_t m = todo[g], run = 0;
+                while (__any(m != 0u)) {
+                    if (m) {
+                        const uint32_t bit = m & (0u - m);
+                        m ^= bit;
+                        const int e = 32 * g + __ffs((int)bit) - 1;
+                        const uint2 ref = list.ref[e];
+                        const int side = strand_side(s, ref, dx, dy, c.float_height);
+                        if (side == 0 || (side < 0 && (ref.y & kStrandNonzero))) run |= bit;
+                        else if (side < 0 && list.box[e].x - dx <= 0.0f) enc ^= 1ull << ((ref.y >> 16) & 63u);
+                    }
+                }
+                todo[g] = run;
+            }
+            for (;;) {
+                int e = -1;
+#pragma unroll
+                for (int g = 0; g < kStrands / 32; ++g)
+                    if (e < 0 && todo[g]) {
+                        e = 32 * g + __ffs((int)todo[g]) - 1;
+                        todo[g] &= todo[g] - 1u;
+                    }
+                if (!__any(e >= 0)) break;
+                if (e < 0) continue;
+                const uint2 ref = list.ref[e];
+                const int k = (int)((ref.y >> 16) & 63u);
+                const bool nonzero = (ref.y & kStrandNonzero) != 0u;
+                if (k != cur) close_winding();
+                const uint32_t label = label_of(k);
+                if ((!kCompact && label >= max_shapes) || q.spilled || q.overflow) continue;
+                const bool reversed = (ref.y & kStrandReversed) != 0u;
+                bool added = false, enclosed = false;
+                emit(ref.x, ref.y, label | (nonzero ? (kNonzero | (reversed ? kReversed : 0u)) : 0u), added, enclosed);
+                if (added) add |= 1ull << k;
+                if (nonzero) {
+                    // a strand crossing the left border above the segment
+                    // adds the sign of its original x direction
+                    any_nonzero = true;
+                    if (cur < 0) { cur = k; w = 0; }
+                    if (enclosed) w += reversed ? -1 : 1;
+                } else if (enclosed) {
+                    enc ^= 1ull << k;
+                }
+            }
+            n = 0;
         }
+        close_winding();
+        if (!alive) enc = 0;
+        uint64_t both = enc | add;
+        if (kCompact) {
+            if (base == 0) { stack0 = enc; contrib0 = both; }
+            else { stack1 = enc; contrib1 = both; }
+            shape_bits += (uint32_t)__popcll(both);
+        } else {
+            while (both && shape_bits < max_shapes) {
+                const int k = __ffsll((long long)both) - 1;
+                both &= both - 1;
+                sidx[(int)shape_bits * kWave] = shape_start + base + k;
+                if ((enc >> k) & 1ull) {
+                    if (shape_bits < 64u) stack0 |= 1ull << shape_bits;
+                    else stack1 |= 1ull << (shape_bits - 64u);
+                }
+                ++shape_bits;
+            }
         }
     }
+    wave_sync();
+}
+
+template <bool kCompact>
+__device__ __forceinline__ void generate(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, bool active, int lane,
+                         float span0, float span1, int32_t *sidx, TileTable *tt,
+                         uint32_t &shape_bits, uint64_t &stack0, uint64_t &stack1,
+                         uint64_t &contrib0, uint64_t &contrib1, bool &any_nonzero)
+{
+    const float dx = (float)c.dx, dy = (float)c.dy;
+    walk_strands<kCompact>(f, s, q, c, active, lane, span0, span1, sidx, tt->strands, shape_bits, stack0, stack1,
+                           contrib0, contrib1, any_nonzero,
+                           [&](uint32_t place, uint32_t meta, uint32_t bit, bool &added, bool &enclosed) {
+                               const GUDNI_CONST uint8_t *strand = ro(s.geo) + 16ull * place;
+                               Trav l = strand_view(strand, dx, dy), r = l;
+                               l.xpos = cl_max(0.0f, l.left.x);
+                               r.xpos = cl_min(1.0f, l.right.x);
+                               search_pair(l, r, strand + 32, ((int)(meta & 0xFFFFu) - 4) / 2, dx, dy);
+                               spawn(q, c, bit, l, r, added, enclosed);
+                           });
 }
 
 // Stable insertion sort by thresholdIsBelow: the same permutation as the
@@ -540,7 +792,6 @@ __device__ void sort_queue(Queue &q)
 // kRadixMin records, or more than half a ring, take the insertion sort
 // alone.
 constexpr int kRadixMin = 8;
-constexpr int kRadixMaxBits = 5;
 
 __device__ __forceinline__ int top_digit(float top, float scale, int nb)
 {
@@ -865,35 +1116,6 @@ __device__ __forceinline__ float4 read_color(const SceneDesc &s, uint64_t tag, i
     return read_color_sub(s, tag, s.substances[tag & kTagIdMask], ax, ay);
 }
 
-// A wave's list of sections waiting for their colours: per section its area
-// (adj) and the stack it lies under, which the colour pass replaces by colour
-// x area.  info: the lane that swept it (bits 0..5), its pixel's row in that
-// lane's segment (6..18), whether it is its pixel's last (kSecEnd), and the
-// lane's next section in the list (24..31, kSecNone: none).
-constexpr int kSections = 192;             // three full waves of colours
-constexpr uint32_t kSecEnd = 1u << 19, kSecNone = 0xFFu;
-struct SectionList {
-    float4 val[kSections];
-    float adj[kSections];
-    uint32_t info[kSections];
-};
-
-// Per-wave LDS table of a compact tile's shapes by tile-local index: tag,
-// and the solid colour (in the coverage mode's form) or, for a picture or
-// gradient, the substance record itself.
-struct TileTable {
-    uint64_t tag[128];
-    float4 color[128];
-    SectionList sec;       // before the sweep: the sort's histogram
-    uint64_t pic0, pic1;   // tile-local shapes whose substance is a picture
-    int grouped;           // the tile qualifies for grouped colours
-    // colour group g holds tile-local shapes [g gq, (g+1) gq), gq = ceil(n / 4)
-    // for a tile of n shapes
-    uint32_t gq;
-};
-static_assert(sizeof(SectionList) >= sizeof(uint16_t) * kWave * (1 << kRadixMaxBits),
-              "the sort histogram lives in the section list");
-
 // Bits [start, start + q) of the 128-bit set (s1:s0), q <= 32, start < 128;
 // bits past 127 read as 0.
 __device__ __forceinline__ uint32_t group_bits(uint64_t s0, uint64_t s1, uint32_t start, uint32_t q)
@@ -1129,13 +1351,6 @@ __device__ __forceinline__ uint32_t pixel_word(float4 c, bool rgba)
     return w;
 }
 
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ void write_pixel(const Frame &f, const SceneDesc &s, int x, int y, float4 color)
 {
     const long long pix = (long long)y * s.width + x;
@@ -1225,7 +1440,7 @@ __device__ __forceinline__ void color_sections(const Frame &f, const SceneDesc &
 // list of 192 keeps five blocks in a CU's LDS: 171 entries take 35.6 ms.
 // Every lane of the wave calls it; ok: the lane has a column to sweep.
 template <bool kCompact>
-__device__ uint32_t render(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, Stack st,
+__device__ __forceinline__ uint32_t render(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, Stack st,
                            int32_t *sidx, TileTable *tt, bool nz, bool ok)
 {
     int32_t *const wind = sidx + kWindOffset * kWave;
@@ -1395,7 +1610,7 @@ __device__ void dump_queue(const Frame &f, const Queue &q, int dslot, bool pre, 
 // with wave-uniform boundaries between the stages so the optional stage
 // clocks bracket whole stages of the wave.
 template <bool kCompact>
-__device__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t unit, Queue &q, int32_t *sidx,
+__device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t unit, Queue &q, int32_t *sidx,
                          TileTable *tt, uint32_t &status)
 {
     const int tile = (int)(unit >> 2), quarter = (int)(unit & 3u);
@@ -1456,13 +1671,13 @@ __device__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t 
         // x extent of this unit's columns (isActiveThread's internalX)
         const int x0 = t.box[0] + unit_x0(t.hdepth, f.compute_depth, quarter);
         const int x1 = x0 + unit_width(t.hdepth, f.compute_depth);
-        generate<kCompact>(f, s, q, c, active, lane, (float)x0 - 1.0f, (float)x1 + 1.0f, sidx, bits,
+        generate<kCompact>(f, s, q, c, active, lane, (float)x0 - 1.0f, (float)x1 + 1.0f, sidx, tt, bits,
                            s0, s1, c0, c1, any_nonzero);
     }
     const bool ok = active && !q.spilled && !q.overflow;
     const long long t1 = timed ? clock64() : 0;
     if (ok && f.dump_qlen) dump_queue<kCompact>(f, q, dslot, true, c0, c1);
-    if (ok) radix_sort_queue(q, reinterpret_cast<uint16_t *>(&tt->sec) + lane, s.sort_bits,
+    if (ok) radix_sort_queue(q, tt->hist + lane, s.sort_bits,
                              c.float_height);
     if (ok && f.dump_qlen) {
         dump_queue<kCompact>(f, q, dslot, false, c0, c1);

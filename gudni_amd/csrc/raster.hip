@@ -37,12 +37,11 @@ namespace dev {
 
 // One persistent pass.  A wave claims a work unit, its lanes run their
 // columns to completion, and the wave loops until the list is empty.
-// The column walks are bound by vector issue and by the latency of their
-// ring and strand reads, so residency pays: five waves per SIMD (at most 96
-// VGPRs, a few spills) render the 4096^2 frame in 35.2 ms; four (no spills)
-// take 35.5 and six (80 VGPRs, a list of 171 sections) 43.6.  Five blocks'
-// tile tables (4 x 7.7 KB each) fit the CU's 160 KB of LDS.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) raster_pass(Frame f, int from_retry)
+// The column walks are bound by vector issue: each wave's own instruction
+// stream takes about ten cycles an instruction, and more waves fill the rest.
+// Four waves per SIMD (at most 128 VGPRs) render the 4096^2 frame in 33.6 ms;
+// five (96 VGPRs, with spills) take 34.2.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) raster_pass(Frame f, int from_retry)
 {
     __shared__ TileTable tables[4];
     const int lane = threadIdx.x & (kWave - 1);
