@@ -168,12 +168,13 @@ struct Frame {
     float4 *q_thr;                // [slots][64][cap]
     uint32_t *q_hdr;              // [slots][64][cap]
     int32_t *shape_idx;           // [slots][max_shapes][64]
-    int32_t cap_log2;
+    int32_t cap_log2, slot_log2;  // records of a lane's ring; of a wave slot's rings
+    int32_t split;                // a unit's 64 columns are run by 2^split waves, 64 >> split lanes each
     // control
     uint32_t *counter;            // work counters of this pass, one per part
     int32_t n_parts;              // parts the work list is cut into
     uint32_t *status;             // OR of lane status flags
-    uint32_t *retry;              // [0] = count, [1..] = abandoned work units
+    uint32_t *retry;              // [0] = count, [1..] = abandoned parts of work units (unit index << split | part)
     int32_t retry_capacity;
     // dump hooks (Level-1 test path), null in normal runs
     float4 *dump_pre_thr; uint32_t *dump_pre_hdr;
@@ -1610,7 +1611,7 @@ __device__ void dump_queue(const Frame &f, const Queue &q, int dslot, bool pre, 
 // with wave-uniform boundaries between the stages so the optional stage
 // clocks bracket whole stages of the wave.
 template <bool kCompact>
-__device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t unit, Queue &q, int32_t *sidx,
+__device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int lane, uint32_t unit, int part, Queue &q, int32_t *sidx,
                          TileTable *tt, uint32_t &status)
 {
     const int tile = (int)(unit >> 2), quarter = (int)(unit & 3u);
@@ -1618,7 +1619,8 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
     const int job = f.tile_job ? f.tile_job[tile] : 0;
     const int column = unit_column(t.hdepth, f.compute_depth, quarter, lane);
     Column c;
-    const bool active = init_column(f, s, t, job, column, c);
+    const bool mine = (lane >> (6 - f.split)) == part;   // a lane of this wave's part of the unit
+    const bool active = init_column(f, s, t, job, column, c) && mine;
     const int dslot = tile * f.threads_per_tile + column;
     const bool timed = f.stage_cycles != nullptr;
     const long long t0 = timed ? clock64() : 0;
@@ -1669,8 +1671,10 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
     bool any_nonzero = false;
     {
         // x extent of this unit's columns (isActiveThread's internalX)
-        const int x0 = t.box[0] + unit_x0(t.hdepth, f.compute_depth, quarter);
-        const int x1 = x0 + unit_width(t.hdepth, f.compute_depth);
+        int x0 = t.box[0] + unit_x0(t.hdepth, f.compute_depth, quarter);
+        const int uw = unit_width(t.hdepth, f.compute_depth), lanes = kWave >> f.split;
+        if (lanes < uw) x0 += (part * lanes) & (uw - 1);
+        const int x1 = x0 + min(uw, lanes);
         generate<kCompact>(f, s, q, c, active, lane, (float)x0 - 1.0f, (float)x1 + 1.0f, sidx, tt, bits,
                            s0, s1, c0, c1, any_nonzero);
     }
@@ -1712,7 +1716,7 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
     // only a lane that walked a nonzero-fill shape keeps winding counters
     status = render<kCompact>(f, s, q, c, Stack{s0, s1}, sidx, tt, any_nonzero, ok);
     if (active && q.overflow) status |= kStatusOverflow;
-    if (!active && f.dump_qlen) f.dump_qlen[dslot] = -1;
+    if (mine && !active && f.dump_qlen) f.dump_qlen[dslot] = -1;
     if (timed) {
         const long long t3 = clock64();
         if (lane == 0) {

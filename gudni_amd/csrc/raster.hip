@@ -9,6 +9,7 @@
 // (unit_column), and units without an active column are never queued (an
 // 8x8 tile is a single unit).  The grid is persistent; every wave loops on an atomic
 // work counter until the list is exhausted, so every wave reaches the exit.
+// A launch of few units splits each among several waves (split_units).
 //
 // Each lane's threshold queue is a ring of its own in the wave slot's
 // scratch.  The fast pass gives each lane a ring of kFastCap records; a lane
@@ -48,17 +49,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) r
     const int wave = threadIdx.x / kWave;
     const int slot = blockIdx.x * (blockDim.x / kWave) + wave;
     const int cap = 1 << f.cap_log2;
-    float4 *q_thr = f.q_thr + ((size_t)slot * kWave + lane) * cap;
-    uint32_t *q_hdr = f.q_hdr + ((size_t)slot * kWave + lane) * cap;
+    const size_t ring = ((size_t)slot << f.slot_log2) + (size_t)(lane & ((kWave >> f.split) - 1)) * cap;
+    float4 *q_thr = f.q_thr + ring;
+    uint32_t *q_hdr = f.q_hdr + ring;
     int32_t *sidx = f.shape_idx + (size_t)slot * kSidxWords * kWave + lane;
     TileTable *tt = &tables[wave];
-    const int n_work = from_retry ? (int)min((uint32_t)f.retry_capacity, f.retry[0]) : f.n_work;
+    const int n_work = from_retry ? (int)min((uint32_t)f.retry_capacity, f.retry[0]) : f.n_work << f.split;
     Claimer claim;
     claim.init(f.counter, f.n_parts, n_work, (int)blockIdx.x);
     for (;;) {
         const int w = claim.next(lane);
         if (w < 0) break;
-        const uint32_t unit = from_retry ? f.retry[1 + w] : f.work[w];
+        const uint32_t item = from_retry ? f.retry[1 + w] : (uint32_t)w;   // unit << split | part
+        const uint32_t unit = f.work[item >> f.split];
+        const int part = (int)(item & ((1u << f.split) - 1u));
         const int count = f.tiles[unit >> 2].shape_count;   // wave-uniform
         const int scene = f.tile_scene
                               ? (int)__builtin_amdgcn_readfirstlane((uint32_t)f.tile_scene[unit >> 2])
@@ -72,16 +76,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) r
         q.head = 0; q.len = 0; q.mask = cap - 1; q.maxt = f.max_thresholds;
         q.spilled = false; q.overflow = false;
         uint32_t status = 0;
-        if (count <= f.max_shapes) run_unit<true>(f, s, lane, unit, q, sidx, tt, status);
-        else run_unit<false>(f, s, lane, unit, q, sidx, tt, status);
+        if (count <= f.max_shapes) run_unit<true>(f, s, lane, unit, part, q, sidx, tt, status);
+        else run_unit<false>(f, s, lane, unit, part, q, sidx, tt, status);
         if (status) atomicOr(f.status, status);
         if (f.scene_done && lane == 0)
             atomicMax(f.scene_done + scene, (unsigned long long)wall_clock64());
-        // a lane whose ring was too small hands the whole unit to the retry pass
+        // a lane whose ring was too small hands the wave's part of the unit to the retry pass
         const bool spilled = __any(q.spilled);
         if (spilled && lane == 0 && !from_retry) {
             const uint32_t k = atomicAdd(f.retry, 1u);
-            if ((int)k < f.retry_capacity) f.retry[1 + k] = unit;
+            if ((int)k < f.retry_capacity) f.retry[1 + k] = item;
             else atomicOr(f.status, kStatusOverflow);
         }
     }
@@ -315,9 +319,36 @@ int ensure_scratch(gudni_ctx *ctx)
     return GUDNI_OK;
 }
 
+// How many waves (2^split, a power of two up to 64) run a unit's 64 columns.
+// A frame of few units leaves most of the chip idle and lasts as long as its
+// slowest unit, and a wave whose columns are tall is slow: its lanes' sweeps
+// diverge, so 64 columns take many times as long as one.  Splitting gives each
+// part a wave (with the slot's rings divided among fewer lanes, each longer,
+// so fewer units are left to the retry pass), at the price of listing the
+// unit's strands once per part.  That price is small where columns are tall
+// and most of the work where they are a row or two, so the number of parts is
+// held to rows / 4 per wave slot, at most 5, for columns of `rows` pixels on
+// average.  On 4096 slots (ms at split 0, 1, ... 6):
+//   641x479, 22 units of 218 rows      3.6 2.8 2.4 2.1 2.0 1.8 1.7   takes 6
+//   64x64, 4 units of 16 rows      .16 .11 .10 .093 .085 .082 .080   takes 6
+//   800x600, 367 units of 20 rows       29  18  13  10 8.3 7.3 6.7   takes 5
+//   1000x701, 536 units of 20 rows      13  11 7.7 5.7 4.3 3.4 4.0   takes 5
+//   768x768, 2 jobs of ~500, 9 rows     18  15  14  12 10. 9.6  11   takes 4
+//   512x512, 4096 units of 1 row        18  20  25  35  56  97 180   takes 0
+//   1920x1080, 8160 units of 4 rows    5.3 5.3 5.8 6.6 8.6  13  22   takes 0
+constexpr int kPartsPerSlot = 5;
+static int split_units(int n_work, double pixels, int slots, int capacity)
+{
+    const double rows = n_work > 0 ? pixels / (64.0 * n_work) : 0.0;
+    const double parts = std::min((double)capacity, slots * std::min((double)kPartsPerSlot, 0.25 * rows));
+    int split = 0;
+    while (split < 6 && (double)n_work * (double)(2 << split) <= parts) ++split;
+    return split;
+}
+
 int ensure_control(gudni_ctx *ctx, int n_work)
 {
-    const int want = std::max(1024, n_work);
+    const int want = std::max(std::max(1024, n_work), kPartsPerSlot * 32 * ctx->cus);   // at most 32 slots a CU
     if (ctx->retry_capacity < want) {
         ++ctx->scratch_gen;
         CHECK_HIP(ctx, ctx->control.ensure(sizeof(uint32_t) * (size_t)(dev::kCtlWords + want)));
@@ -407,7 +438,8 @@ static PassBuffers ctx_buffers(gudni_ctx *ctx)
                        ctx->slow_blocks, 256};
 }
 
-static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b)
+// pixels: what the launch covers, for the choice of the split.
+static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, double pixels)
 {
     uint32_t *ctl = b.ctl;
     hipLaunchKernelGGL(dev::reset_counters, dim3(1), dim3(64), 0, ctx->stream, ctl, dev::kCtlWords);
@@ -422,26 +454,32 @@ static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b)
     f.q_thr = b.fast_thr;
     f.q_hdr = b.fast_hdr;
     f.shape_idx = b.fast_sidx;
-    f.cap_log2 = dev::kFastCapLog2;
-    const int fast_grid = std::max(1, std::min(b.fast_blocks, (f.n_work + 3) / 4));
+    int slog = 0;
+    while ((1 << slog) < ctx->spec.max_thresholds) ++slog;
+    f.split = split_units(f.n_work, pixels, 4 * b.fast_blocks, b.retry_capacity);
+    f.slot_log2 = dev::kFastCapLog2 + 6;
+    f.cap_log2 = std::min(dev::kFastCapLog2 + f.split, std::max(slog, dev::kFastCapLog2));
+    const int fast_grid = std::max(1, std::min(b.fast_blocks, ((f.n_work << f.split) + 3) / 4));
     hipLaunchKernelGGL(dev::raster_pass, dim3(fast_grid), dim3(256), 0, ctx->stream, f, 0);
     CHECK_HIP(ctx, hipGetLastError());
     if (ctx->timed_render) CHECK_HIP(ctx, hipEventRecord(ctx->ev[1], ctx->stream));
     // retry pass: rings of maxThresholds records
-    int slog = 0;
-    while ((1 << slog) < ctx->spec.max_thresholds) ++slog;
     f.counter = ctl + dev::kCtlSlow;
     f.n_parts = 1;
     f.q_thr = b.slow_thr;
     f.q_hdr = b.slow_hdr;
     f.shape_idx = b.slow_sidx;
     f.cap_log2 = slog;
+    f.slot_log2 = slog + 6;
     hipLaunchKernelGGL(dev::raster_pass, dim3(b.slow_blocks), dim3(b.slow_threads), 0, ctx->stream, f, 1);
     CHECK_HIP(ctx, hipGetLastError());
     return GUDNI_OK;
 }
 
-static int launch_passes(gudni_ctx *ctx, dev::Frame f) { return launch_passes(ctx, f, ctx_buffers(ctx)); }
+static int launch_passes(gudni_ctx *ctx, dev::Frame f, double pixels)
+{
+    return launch_passes(ctx, f, ctx_buffers(ctx), pixels);
+}
 
 int read_status(gudni_ctx *ctx)
 {
@@ -1039,7 +1077,13 @@ static int run_job(gudni_ctx *ctx, const void *shapes, int32_t n_shapes, const v
         f.dump_cap = (int32_t)cap;
     }
     ctx->timed_render = false;
-    rc = launch_passes(ctx, f);
+    double pixels = 0.0;
+    for (int32_t t = 0; t < n_tiles; ++t) {
+        const TileRec &r = ((const TileRec *)tiles)[t];
+        pixels += std::max(0.0, std::min(w, r.box[2]) - (double)r.box[0]) *
+                  std::max(0.0, std::min(h, r.box[3]) - (double)r.box[1]);
+    }
+    rc = launch_passes(ctx, f, pixels);
     if (rc) return rc;
     rc = read_status(ctx);
     if (rc) return rc;
@@ -1158,7 +1202,7 @@ int gudni_frame_render(gudni_ctx *ctx, uint32_t *out_dev, float *out_f32_dev)
         CHECK_HIP(ctx, hipEventRecord(ctx->ev[0], ctx->stream));
     }
     ctx->timed_render = ctx->timing;
-    int rc = launch_passes(ctx, f);
+    int rc = launch_passes(ctx, f, (double)ctx->frame_w * ctx->frame_h);
     if (rc) return rc;
     if (ctx->timing) CHECK_HIP(ctx, hipEventRecord(ctx->ev[2], ctx->stream));
     return GUDNI_OK;
@@ -1205,7 +1249,7 @@ int gudni_frame_render_static(gudni_ctx *ctx, uint32_t *out_dev, float *out_f32_
                         reinterpret_cast<float4 *>(base + kOffSlowThr),
                         reinterpret_cast<uint32_t *>(base + kOffSlowHdr),
                         reinterpret_cast<int32_t *>(base + kOffSlowSidx), 1, 64};
-    return launch_passes(ctx, f, b);
+    return launch_passes(ctx, f, b, (double)ctx->frame_w * ctx->frame_h);
 }
 
 int gudni_frame_check(gudni_ctx *ctx)
@@ -1768,7 +1812,9 @@ static int batch_launch(gudni_ctx *ctx, gudni_batch *b)
     hipLaunchKernelGGL(dev::batch_begin, dim3(blocks), dim3(threads), 0, ctx->stream,
                        (unsigned long long *)b->done.p, b->n_scenes);
     CHECK_HIP(ctx, hipGetLastError());
-    return launch_passes(ctx, batch_frame(ctx, b));
+    double pixels = 0.0;
+    for (int32_t s = 0; s < b->n_scenes; ++s) pixels += (double)b->width[s] * b->height[s];
+    return launch_passes(ctx, batch_frame(ctx, b), pixels);
 }
 
 int gudni_batch_render(gudni_ctx *ctx, gudni_batch *b, int use_graph)
@@ -1831,7 +1877,7 @@ int gudni_batch_render_scene(gudni_ctx *ctx, gudni_batch *b, int32_t scene)
     f.work = (const uint32_t *)b->work.p + b->work_begin[scene];
     f.n_work = b->work_count[scene];
     f.scene_done = nullptr;
-    return launch_passes(ctx, f);
+    return launch_passes(ctx, f, (double)b->width[scene] * b->height[scene]);
 }
 
 int gudni_batch_check(gudni_ctx *ctx, gudni_batch *b, float *latency_ms)

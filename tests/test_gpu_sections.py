@@ -38,3 +38,29 @@ def test_section_lists(n, width, height, mode):
         r.close()
     assert np.array_equal(got, want["out"]), H.first_mismatch(got, want["out"])
     assert np.array_equal(f32, want["f32"])
+
+
+@pytest.mark.parametrize("tile,width,height", [(32, 512, 768), (32, 300, 257), (64, 200, 130), (256, 40, 300), (16, 64, 33)])
+def test_units_split_over_waves(tile, width, height):
+    """Frames of few units run each unit in 1 to 64 waves, by their number and
+    height; one pixel column holds more records than any of the small rings,
+    so parts of units go through the retry pass."""
+    bars = [S.rectangle_pairs(20 + (2 * i + 0.5) / 300, -1.0, 20 + (2 * i + 1.5) / 300, height + 1.0) for i in range(150)]
+    rng = np.random.default_rng(width)
+    shapes, cols = [(S.solid_tag(0), bars)], [[0.9, 0.2, 0.1, 0.6]]
+    for i in range(1, 40):
+        p = rng.uniform(0, 1, (int(rng.integers(3, 7)), 4)) * [width, height, width, height]
+        shapes.append((S.nonzero(S.solid_tag(i)) if i % 3 == 0 else S.solid_tag(i), [p]))
+        cols.append(rng.uniform(0, 1, 4))
+    scene = S.build_scene(width, height, shapes, cols, name="split")
+    spec = G.default_spec(max_tile_size=tile)
+    want = H.oracle_render(scene, spec, want_f64=False)
+    assert want["rc"] == 0
+    r = G.Rasterizer(spec)
+    try:
+        got, f32 = H.gpu_render_level2(r, scene, spec)
+        assert np.array_equal(got, want["out"]), H.first_mismatch(got, want["out"])
+        assert np.array_equal(f32, want["f32"])
+        assert np.array_equal(H.gpu_render_level1(r, scene, spec), want["out"])
+    finally:
+        r.close()
