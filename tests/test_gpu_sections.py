@@ -64,3 +64,34 @@ def test_units_split_over_waves(tile, width, height):
         assert np.array_equal(H.gpu_render_level1(r, scene, spec), want["out"])
     finally:
         r.close()
+
+
+@pytest.mark.parametrize("copies,nonzero", [(1, False), (2, False), (5, True), (40, False)])
+def test_records_that_tie(copies, nonzero):
+    """Edges that several shapes share, edges that meet at one height and
+    edges that cross: the lower parts of split records go back among records
+    they tie with, in the reference's order."""
+    w, h = 21, 19
+    quads = [[(2.5, 1.0), (15.25, 4.0), (9.0, 17.5), (1.0, 12.0)], [(15.25, 4.0), (20.0, 4.0), (20.0, 12.0), (9.0, 17.5)],
+             [(0.0, 4.0), (20.5, 4.0), (20.5, 8.0), (0.0, 8.0)], [(3.0, 2.0), (17.0, 16.0), (3.0, 16.0), (17.0, 2.0)],
+             [(5.0, 0.5), (5.0, 18.5), (6.0, 18.5), (6.0, 0.5)]]
+    rng = np.random.default_rng(copies)
+    shapes, cols = [], []
+    for k in range(copies):
+        for i, p in enumerate(quads):
+            tag = S.solid_tag(len(shapes))
+            shapes.append((S.nonzero(tag) if nonzero and (i + k) % 2 else tag, [S.straight_pairs(p)]))
+            cols.append(rng.uniform(0, 1, 4))
+    scene = S.build_scene(w, h, shapes, cols, name="ties")
+    for tile in (8, 256):
+        for mode in (0, 1):
+            spec = G.default_spec(max_tile_size=tile, coverage_mode=mode)
+            want = H.oracle_render(scene, spec, want_f64=False)
+            assert want["rc"] == 0
+            r = G.Rasterizer(spec)
+            try:
+                got, f32 = H.gpu_render_level2(r, scene, spec)
+            finally:
+                r.close()
+            assert np.array_equal(got, want["out"]), H.first_mismatch(got, want["out"])
+            assert np.array_equal(f32, want["f32"])
