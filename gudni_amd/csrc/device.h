@@ -449,7 +449,7 @@ struct TileTable {
         StrandList strands;    // generation's strands
         uint16_t hist[(1 << kRadixMaxBits) * kWave];   // the sort's histogram
     };
-    uint64_t pic0, pic1;   // tile-local shapes whose substance is a picture
+    int mixed;             // some shape is a picture or gradient (adjoint)
     int grouped;           // the tile qualifies for grouped colours
     // colour group g holds tile-local shapes [g gq, (g+1) gq), gq = ceil(n / 4)
     // for a tile of n shapes
@@ -1262,48 +1262,11 @@ __device__ __forceinline__ float4 grouped_color(const SceneDesc &s, const TileTa
     return make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// A lane's colours of the current pixel for picture and gradient layers of a
-// compact tile, which depend on the shape and the pixel only: the tile's
-// first 32 such shapes (by rank among them, tt->pic0/pic1) keep theirs in
-// the first 128 words of the lane's shape scratch, which a compact tile
-// does not use.  known: which ranks hold the current pixel's colour (clear
-// it at every new pixel).
-struct LayerCache {
-    int32_t *words;
-    uint32_t known;
-
-    __device__ __forceinline__ float4 color(const SceneDesc &s, const TileTable *tt, int n, uint64_t tag,
-                                            float4 sub, int ax, int ay)
-    {
-        const uint64_t pm0 = tt->pic0, pm1 = tt->pic1;
-        const uint32_t rank =
-            n < 64 ? (uint32_t)__popcll(pm0 & ((1ull << n) - 1ull))
-                   : (uint32_t)(__popcll(pm0) + __popcll(pm1 & ((1ull << (n - 64)) - 1ull)));
-        if (rank < 32u && ((known >> rank) & 1u))
-            return make_float4(__int_as_float(words[(4 * rank + 0) * kWave]),
-                               __int_as_float(words[(4 * rank + 1) * kWave]),
-                               __int_as_float(words[(4 * rank + 2) * kWave]),
-                               __int_as_float(words[(4 * rank + 3) * kWave]));
-        const float4 c = read_color_sub(s, tag, sub, ax, ay);
-        if (rank < 32u) {
-            words[(4 * rank + 0) * kWave] = __float_as_int(c.x);
-            words[(4 * rank + 1) * kWave] = __float_as_int(c.y);
-            words[(4 * rank + 2) * kWave] = __float_as_int(c.z);
-            words[(4 * rank + 3) * kWave] = __float_as_int(c.w);
-            known |= 1u << rank;
-        }
-        return c;
-    }
-};
-
 // determineColor (Kernels.cl:1447-1513).  kCompact: the stack is labelled by
-// tile-local shape index and tags/colours come from the LDS table.  lc (a
-// compact tile's, or null): picture and gradient colours through the lane's
-// cache of the current pixel.
+// tile-local shape index and tags/colours come from the LDS table.
 template <bool kCompact>
 __device__ float4 determine_color(const Frame &f, const SceneDesc &s, const Stack &st, const int32_t *sidx,
-                                  const TileTable *tt, int ax, int ay, bool &positional,
-                                  LayerCache *lc = nullptr)
+                                  const TileTable *tt, int ax, int ay)
 {
     // The walk visits set stack bits from the top (findTop with a falling
     // ignoreAbove, Kernels.cl:281-292): pop the highest bit of a working copy.
@@ -1344,12 +1307,8 @@ __device__ float4 determine_color(const Frame &f, const SceneDesc &s, const Stac
                 if (kCompact && solid) {
                     next = tt->color[top_bit];          // already in the mode's form
                 } else {
-                    if (kCompact)
-                        next = lc ? lc->color(s, tt, top_bit, tag, tt->color[top_bit], ax, ay)
-                                  : read_color_sub(s, tag, tt->color[top_bit], ax, ay);
-                    else
-                        next = read_color(s, tag, ax, ay);
-                    positional = positional || !solid;
+                    if (kCompact) next = read_color_sub(s, tag, tt->color[top_bit], ax, ay);
+                    else next = read_color(s, tag, ax, ay);
                     if (!ref_mode)
                         next = make_float4(next.x * next.w, next.y * next.w, next.z * next.w, next.w);
                 }
@@ -1431,9 +1390,7 @@ __device__ __forceinline__ void color_sections(const Frame &f, const SceneDesc &
         if (grouped) {
             col = grouped_color(s, tt, s0, s1, valid, ax, ay);
         } else {
-            bool positional = false;
-            if (valid)
-                col = determine_color<kCompact>(f, s, Stack{s0, s1}, sidx - lane + owner, tt, ax, ay, positional);
+            if (valid) col = determine_color<kCompact>(f, s, Stack{s0, s1}, sidx - lane + owner, tt, ax, ay);
         }
         if (valid) {
             const float adj = L.adj[e];
@@ -1688,7 +1645,6 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
         // the tile's tags and solid colours, by tile-local index
         const bool premultiply = f.coverage_mode != GUDNI_COVERAGE_REFERENCE;
         bool all_add = true;
-        uint64_t pic_lo = 0, pic_hi = 0;
         for (int n = lane; n < c.num_shapes; n += kWave) {
             const uint64_t tag = s.shapes[c.shape_start + n].tag;
             tt->tag[n] = tag;
@@ -1705,19 +1661,9 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
             const uint64_t sid = tt->tag[n] & kTagIdMask;
             for (int m = n + 1; m < c.num_shapes && distinct; ++m)
                 distinct = (tt->tag[m] & kTagIdMask) != sid;
-            if ((tt->tag[n] & kTagTypeMask) != kTagSolid) {
-                if (n < 64) pic_lo |= 1ull << n; else pic_hi |= 1ull << (n - 64);
-            }
-        }
-        // OR-reduce the picture masks and AND-reduce the flags over the wave
-        for (int o = 32; o > 0; o >>= 1) {
-            pic_lo |= __shfl_xor(pic_lo, o);
-            pic_hi |= __shfl_xor(pic_hi, o);
         }
         const bool grouped_tile = premultiply && __all(all_add && distinct);
         if (lane == 0) {
-            tt->pic0 = pic_lo;
-            tt->pic1 = pic_hi;
             tt->grouped = grouped_tile ? 1 : 0;
             const uint32_t gq = c.num_shapes > 4 ? (uint32_t)(c.num_shapes + 3) / 4u : 1u;
             tt->gq = gq;

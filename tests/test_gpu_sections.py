@@ -95,3 +95,37 @@ def test_records_that_tie(copies, nonzero):
                 r.close()
             assert np.array_equal(got, want["out"]), H.first_mismatch(got, want["out"])
             assert np.array_equal(f32, want["f32"])
+
+
+@pytest.mark.parametrize("height,tile", [(1, 16), (51, 64), (52, 64), (120, 256), (256, 256)])
+def test_adjoint_keeps_section_colours(height, tile):
+    """Columns of fewer and more sections (5 a pixel) than the colours a lane
+    keeps for the backward sweep (256): colour gradients of bars that do not
+    overlap, over an opaque background, equal their closed form in FP64.
+    Tolerance: 2 x 256 x 3 terms of either sign added in FP32, 2^-24 each."""
+    w = 3
+    a, b = [], []
+    for x in range(w):
+        a.append(S.rectangle_pairs(x + 0.125, -1.0, x + 0.375, height + 1.0))
+        b.append(S.rectangle_pairs(x + 0.5, -1.0, x + 0.875, height + 1.0))
+    cols = np.array([[0.9, 0.2, 0.1, 0.625], [0.1, 0.4, 0.8, 0.75]], np.float32)
+    scene = S.build_scene(w, height, [(S.solid_tag(0), a), (S.solid_tag(1), b)], cols, name="bars")
+    target = np.random.default_rng(height).uniform(0, 1, (height, w, 4)).astype(np.float32)
+    r = G.Rasterizer(G.default_spec(max_tile_size=tile))
+    try:
+        adj = G.Adjoint(r, [(scene, target)])
+        adj.run()
+        loss, _, d_rgba, image = adj.result(0, image=True)
+        adj.close()
+    finally:
+        r.close()
+    c, cov, bg = cols.astype(np.float64), np.array([0.25, 0.375]), np.ones(3)
+    over = c[:, :3] * c[:, 3:] + bg * (1.0 - c[:, 3:])
+    rgb = cov @ over + (1.0 - cov.sum()) * bg
+    assert np.abs(image[..., :3] - rgb).max() < 1e-6
+    err = rgb - target[..., :3].astype(np.float64)
+    g = 2.0 * err.sum(axis=(0, 1))
+    want = np.concatenate([cov[:, None] * c[:, 3:] * g, (cov[:, None] * (c[:, :3] - bg) * g).sum(axis=1, keepdims=True)], axis=1)
+    bound = 2.0 ** -24 * 2 * 256 * 3 * 2.0 * np.abs(err).sum()
+    assert np.abs(d_rgba - want).max() <= max(bound, 1e-6)
+    assert abs(loss - ((err ** 2).sum() + ((1.0 - target[..., 3].astype(np.float64)) ** 2).sum())) <= 1e-5 * loss
