@@ -1512,6 +1512,8 @@ int scene_ser_in(gudni_ctx *ctx, gudni_adjoint_batch *a, int s, SerIn &in)
     in.ooff = (const int32_t *)v.ooff.p;
     in.pairs = (const float *)a->points.p + 2 * a->points_off[s];
     in.n_shapes = n;
+    in.n_outlines = (int32_t)sc.outline_off.size() - 1;
+    in.n_pairs = (int32_t)(sc.pairs.size() / 4);
     in.width = sc.width;
     in.height = sc.height;
     in.subs = (const float4 *)a->subs.p + a->subs_off[s];

@@ -160,11 +160,14 @@ __device__ void init_body(const Dev &d, int t0, int ts)
 
 __global__ void __launch_bounds__(kThreads) bin_init(Dev d) { init_body(d, gtid(), gstride()); }
 
+// Eight lanes a node (they add its shapes' strands together: one lane's chain
+// of up to 126 dependent reads was most of a small scene's build).
 __device__ void decide_body(const Dev &d, const ShapeRec *shapes, int level, int t0, int ts)
 {
     if (d.status[0]) return;
     const int4 lv = d.levels[level];
-    for (int i = t0; i < lv.y; i += ts) {
+    const int sub = t0 & 7;
+    for (int i = t0 >> 3; i < lv.y; i += ts >> 3) {
         const int n = lv.x + i;
         const int4 m = d.node_meta[n];
         uint32_t flags = (uint32_t)m.y;
@@ -180,13 +183,16 @@ __device__ void decide_body(const Dev &d, const ShapeRec *shapes, int level, int
                 split = true;
             } else {
                 uint64_t s = 0;
-                for (int k = 0; k < m.w; ++k) s += shapes[d.pair_shape[m.z + k]].num_strands;
+                for (int k = sub; k < m.w; k += 8) s += shapes[d.pair_shape[m.z + k]].num_strands;
+                for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o);
                 split = !(s < (uint64_t)d.p.cap_strands);
             }
         }
         if (split) flags |= kFlagSplit;
-        d.node_meta[n].y = (int)flags;
-        d.node_child[n] = -1;
+        if (sub == 0) {
+            d.node_meta[n].y = (int)flags;
+            d.node_child[n] = -1;
+        }
     }
 }
 

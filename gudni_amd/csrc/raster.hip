@@ -636,8 +636,38 @@ int validate_job(gudni_ctx *ctx, const CommonView &cv, const ShapeRec *shapes,
     return GUDNI_OK;
 }
 
+// Whether one block builds a scene's tree sooner than the level launches,
+// which cost 0.6 to 0.9 ms (some 200 of them) however little there is to do.
+// `cells`: the root's forced leaves.  The block's time goes with the pairs it
+// moves, at most shapes x cells a level.  Measured (us, block against
+// launches): 250^2, 120 shapes, 16-px tiles (256 cells) 130 / 569; 640^2, 300,
+// 256 px (16) 108 / 825; 512^2, 1,000, 32 px (256) 344 / 675; 800^2, 3,000,
+// 256 px (16) 529 / 823; 1920^2, 1,000, 64 px (1,024) 764 / 963; beyond the
+// line 512^2, 2,000, 16 px (1,024) 1,047 / 685.
+static bool one_block_scene(int64_t shapes, int64_t cells)
+{
+    return shapes <= 4096 && cells <= 1024 && shapes * cells <= (1 << 20);
+}
+
 int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt)
 {
+    const int side = ceil_log2(std::max(in.width, in.height)) -
+                     ceil_log2(in.max_tile_size > 0 ? in.max_tile_size : ctx->spec.max_tile_size);
+    if (one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side))) {
+        if (ctx->timing) {
+            for (hipEvent_t &e : ctx->bin_ev)
+                if (!e) CHECK_HIP(ctx, hipEventCreate(&e));
+            CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[0], ctx->stream));
+        }
+        const int rc = bin_scenes(ctx, &in, &out, &cnt, 1);
+        if (rc) return rc;
+        if (ctx->timing) {
+            CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[1], ctx->stream));
+            CHECK_HIP(ctx, hipEventSynchronize(ctx->bin_ev[1]));
+            CHECK_HIP(ctx, hipEventElapsedTime(&ctx->last_bin_ms, ctx->bin_ev[0], ctx->bin_ev[1]));
+        }
+        return GUDNI_OK;
+    }
     binning::Params bp;
     bp.n_shapes = in.n_shapes;
     bp.canvas_depth = ceil_log2(std::max(in.width, in.height));
@@ -1698,6 +1728,8 @@ int gudni_batch_upload_outlines(gudni_ctx *ctx, int32_t n_scenes, const gudni_ou
         in.ooff = (const int32_t *)ctx->ser_ooff.p;
         in.pairs = (const float *)ctx->ser_pairs.p;
         in.n_shapes = n;
+        in.n_outlines = n_outlines;
+        in.n_pairs = n_pairs;
         in.width = sc.width;
         in.height = sc.height;
         in.subs = (const float4 *)b->subs.p + subs_off[s];

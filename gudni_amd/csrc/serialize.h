@@ -10,7 +10,7 @@ struct SerIn {
     const uint64_t *tags;          // device: per shape
     const int32_t *soff, *ooff;    // device: shape -> outlines, outline -> pairs
     const float *pairs;            // device: [n_pairs][4]
-    int32_t n_shapes;
+    int32_t n_shapes, n_outlines, n_pairs;
     int32_t width, height;
     const float4 *subs;            // device substance table (substance checks)
     int32_t n_subs, n_uses, n_grads;

@@ -6,8 +6,12 @@
 // ReorderTable.hs:44-111, Serialize.hs:76-177, Outline.hs:123-133) with the
 // same FP32 operations in the same order, so the bytes are the same.
 //
-// Layout of the work: one thread per shape (shapes hold a few outlines of
-// 3..30 pairs; the walk over a shape's curves is short and serial).
+// Layout of the work:
+//   knobs     one thread per curve pair: where its knob is split, if it has one
+//             (a bisection of up to 14 dependent steps, the longest chain of
+//             the serialiser)
+// then one thread per shape (shapes hold a few outlines of 3..30 pairs; with
+// the knobs known the walk over a shape's curves is short and serial):
 //   count     box, cull, substance checks, and per outline a streaming pass
 //             over its knob-split curves that sizes every run of one x
 //             direction (16-byte units and strands) in O(1) state
@@ -50,7 +54,8 @@ struct Args {
     const uint64_t *tags;
     const int32_t *soff, *ooff;
     const float *pairs;
-    int32_t n_shapes;
+    int32_t n_shapes, n_outlines, n_pairs;
+    float *knob;                // per pair: its curve's split parameter, or kNoKnob
     float fw, fh;
     const float4 *subs;
     int32_t n_subs, n_uses, n_grads;
@@ -74,22 +79,15 @@ __device__ __forceinline__ Pt lerp_t(float t, Pt a, Pt b)
 // A control point strictly outside the end points' x range is a knob: split
 // where dx/dt changes sign, found by bisection on FP32 parameters to
 // iota = 1e-4 (Deknob.hs:61-79, Figure/Space.hs:101-102).
-__device__ int split_knob(const Quad &q, Quad *out, float &split_t)
+constexpr float kNoKnob = -1.0f;
+__device__ float find_knob(const Quad &q)
 {
     const bool bulge_left = q.c.x < q.p0.x && q.c.x < q.p1.x;
     const bool bulge_right = q.c.x > q.p0.x && q.c.x > q.p1.x;
-    split_t = 0.0f;
-    if (!bulge_left && !bulge_right) {
-        out[0] = q;
-        return 1;
-    }
+    if (!bulge_left && !bulge_right) return kNoKnob;
     float lo = 0.0f, hi = 1.0f, t = 0.5f;
-    Pt m0, on, m1;
-    for (;;) {
-        m0 = lerp_t(t, q.p0, q.c);
-        m1 = lerp_t(t, q.c, q.p1);
-        on = lerp_t(t, m0, m1);
-        if (hi - lo <= 0.0001f) break;
+    while (!(hi - lo <= 0.0001f)) {
+        const Pt m0 = lerp_t(t, q.p0, q.c), m1 = lerp_t(t, q.c, q.p1), on = lerp_t(t, m0, m1);
         const bool out1 = bulge_left ? m1.x < on.x : m1.x > on.x;
         const bool out0 = bulge_left ? m0.x < on.x : m0.x > on.x;
         if (out1) {                // still bulging: move toward p1
@@ -104,9 +102,19 @@ __device__ int split_knob(const Quad &q, Quad *out, float &split_t)
             break;
         }
     }
+    return t;
+}
+
+// The curve's halves at its knob, or the curve.
+__device__ __forceinline__ int split_knob(const Quad &q, float t, Quad *out)
+{
+    if (t == kNoKnob) {
+        out[0] = q;
+        return 1;
+    }
+    const Pt m0 = lerp_t(t, q.p0, q.c), m1 = lerp_t(t, q.c, q.p1), on = lerp_t(t, m0, m1);
     out[0] = Quad{q.p0, m0, on};
     out[1] = Quad{on, m1, q.p1};
-    split_t = t;
     return 2;
 }
 
@@ -138,7 +146,7 @@ struct Runs {
 
 // Maximal runs of knob-free curves sharing a non-zero x direction (a
 // vertical curve is a run of its own).
-__device__ Runs count_runs(const float *p, int k)
+__device__ Runs count_runs(const float *p, const float *knob, int k)
 {
     Runs r{0u, 0u, 0u, 0u, 0u};
     if (k < 2) return r;
@@ -146,8 +154,7 @@ __device__ Runs count_runs(const float *p, int k)
     uint32_t len = 0, start = 0, idx = 0;
     for (int i = 0; i < k; ++i) {
         Quad two[2];
-        float t;
-        const int n = split_knob(curve_at(p, i, k), two, t);
+        const int n = split_knob(curve_at(p, i, k), knob[i], two);
         for (int h = 0; h < n; ++h, ++idx) {
             const int d = x_dir(two[h]);
             if (idx == 0) {
@@ -203,7 +210,7 @@ __device__ void write_strand(const Quad *buf, int m, uint8_t *dst, const Orders 
 // Writes one outline's strands from heap unit `base` on; with tracking,
 // their curves' records from curve `cbase` on (pair_base: the outline's
 // first pair in the scene).
-__device__ void emit_outline(const float *p, int k, const Runs &r, uint8_t *heap, uint64_t base,
+__device__ void emit_outline(const float *p, const float *knob, int k, const Runs &r, uint8_t *heap, uint64_t base,
                              const Orders &ord, CurveSrc *curves, uint64_t cbase, int32_t pair_base,
                              bool mark_reversed)
 {
@@ -234,8 +241,8 @@ __device__ void emit_outline(const float *p, int k, const Runs &r, uint8_t *heap
     };
     for (int i = 0; i < k; ++i) {
         Quad two[2];
-        float t;
-        const int n = split_knob(curve_at(p, i, k), two, t);
+        const float t = knob[i];
+        const int n = split_knob(curve_at(p, i, k), t, two);
         const int j = (i + 1 == k) ? 0 : i + 1;
         const int32_t a = 2 * (pair_base + i), b = 2 * (pair_base + j);
         for (int h = 0; h < n; ++h, ++idx) {
@@ -252,7 +259,7 @@ __device__ void emit_outline(const float *p, int k, const Runs &r, uint8_t *heap
             }
             buf[nb] = two[h];
             if (curves)
-                src[nb] = CurveSrc{a, a + 1, b, t, n == 2 ? (h == 0 ? kCurveLowerHalf : kCurveUpperHalf) : 0u};
+                src[nb] = CurveSrc{a, a + 1, b, n == 2 ? t : 0.0f, n == 2 ? (h == 0 ? kCurveLowerHalf : kCurveUpperHalf) : 0u};
             ++nb;
         }
     }
@@ -265,6 +272,22 @@ __device__ __forceinline__ int gstride() { return (int)(gridDim.x * blockDim.x);
 // Kernel bodies over (first thread, stride): the single-scene kernels run
 // them over the grid, the many-scene kernels over the blocks of a grid row
 // (blockIdx.y = scene).
+__device__ void knobs_body(const Args &a, int t0, int ts)
+{
+    for (int i = t0; i < a.n_pairs; i += ts) {
+        // the outline that holds pair i: the last that starts at or before it
+        int lo = 0, hi = a.n_outlines;
+        while (hi - lo > 1) {
+            const int m = (lo + hi) >> 1;
+            if (a.ooff[m] <= i) lo = m;
+            else hi = m;
+        }
+        const int e0 = a.ooff[lo], e1 = a.ooff[lo + 1];
+        if (i < e0 || i >= e1) continue;
+        a.knob[i] = find_knob(curve_at(a.pairs + 4 * (size_t)e0, i - e0, e1 - e0));
+    }
+}
+
 __device__ void count_body(const Args &a, int t0, int ts)
 {
     for (int s = t0; s < a.n_shapes; s += ts) {
@@ -312,7 +335,7 @@ __device__ void count_body(const Args &a, int t0, int ts)
             }
             for (int o = o0; o < o1; ++o) {
                 const int e0 = a.ooff[o], e1 = a.ooff[o + 1];
-                const Runs rr = count_runs(a.pairs + 4 * (size_t)e0, e1 - e0);
+                const Runs rr = count_runs(a.pairs + 4 * (size_t)e0, a.knob + e0, e1 - e0);
                 units += rr.units;
                 strands += rr.strands;
             }
@@ -335,8 +358,8 @@ __device__ void emit_body(const Args &a, const Orders &ord, int t0, int ts)
         for (int o = o0; o < o1; ++o) {
             const int e0 = a.ooff[o], e1 = a.ooff[o + 1];
             const float *p = a.pairs + 4 * (size_t)e0;
-            const Runs rr = count_runs(p, e1 - e0);
-            emit_outline(p, e1 - e0, rr, a.heap, base, ord, a.curves, cbase, e0,
+            const Runs rr = count_runs(p, a.knob + e0, e1 - e0);
+            emit_outline(p, a.knob + e0, e1 - e0, rr, a.heap, base, ord, a.curves, cbase, e0,
                          (a.tags[s] & dev::kTagNonzero) != 0);
             base += rr.units;
             cbase += rr.units - rr.strands;
@@ -378,6 +401,21 @@ __device__ void extents_body(const Args &a, int n, int t0, int ts)
     }
 }
 
+__global__ void __launch_bounds__(kThreads) ser_knobs(Args a)
+{
+    if (gtid() < 4) a.status[gtid()] = 0u;
+    knobs_body(a, gtid(), gstride());
+}
+
+// The sizes and the status in one place, for one copy to the host.
+__global__ void ser_totals(Args a, uint64_t *totals)
+{
+    totals[0] = a.kidx[a.n_shapes];
+    totals[1] = a.ustart[a.n_shapes];
+    totals[2] = a.cstart ? a.cstart[a.n_shapes] : 0;
+    totals[3] = a.status[0];
+}
+
 __global__ void __launch_bounds__(kThreads) ser_count(Args a) { count_body(a, gtid(), gstride()); }
 
 __global__ void __launch_bounds__(kThreads) ser_emit(Args a, Orders ord) { emit_body(a, ord, gtid(), gstride()); }
@@ -387,15 +425,14 @@ __global__ void __launch_bounds__(kThreads) ser_extents(Args a, const uint64_t *
     extents_body(a, (int)*n_kept, gtid(), gstride());
 }
 
-__global__ void ser_reset(uint32_t *status) { if (threadIdx.x < 4) status[threadIdx.x] = 0u; }
-
 __device__ __forceinline__ int row_tid() { return (int)(blockIdx.x * blockDim.x + threadIdx.x); }
 __device__ __forceinline__ int row_stride() { return (int)(gridDim.x * blockDim.x); }
 
-__global__ void ser_reset_many(const Args *args, int n)
+__global__ void __launch_bounds__(kThreads) ser_knobs_many(const Args *args)
 {
-    for (int s = row_tid(); s < n; s += row_stride())
-        for (int k = 0; k < 4; ++k) args[s].status[k] = 0u;
+    const Args &a = args[blockIdx.y];
+    if (row_tid() < 4) a.status[row_tid()] = 0u;
+    knobs_body(a, row_tid(), row_stride());
 }
 
 __global__ void __launch_bounds__(kThreads) ser_count_many(const Args *args)
@@ -505,10 +542,10 @@ int serialize_outlines(gudni_ctx *ctx, const SerIn &in, const SerOut &out, SerCo
     const hipStream_t st = ctx->stream;
     const int32_t n = in.n_shapes;
     CHECK_HIP(ctx, ctx->ser_work.ensure(16u * (size_t)n + 8u * (4 * (size_t)n + 3) + 4u * 2 * (size_t)n +
-                                        8u * (devscan::kScanBlocks + 1) + 64));
+                                        4u * (size_t)in.n_pairs + 8u * (devscan::kScanBlocks + 1) + 96));
     ser::Args a;
     std::memset(&a, 0, sizeof(a));
-    uint64_t *partials;
+    uint64_t *partials, *totals_dev;
     {
         // float4 first, then 8-byte and 4-byte arrays: every array aligned
         uint8_t *w = (uint8_t *)ctx->ser_work.p;
@@ -519,8 +556,10 @@ int serialize_outlines(gudni_ctx *ctx, const SerIn &in, const SerOut &out, SerCo
         a.cstart = (uint64_t *)w;         w += 8u * ((size_t)n + 1);
         a.keep = (uint32_t *)w;           w += 4u * (size_t)n;
         a.strands = (uint32_t *)w;        w += 4u * (size_t)n;
+        a.knob = (float *)w;              w += 4u * (size_t)in.n_pairs;
         a.status = (uint32_t *)w;         w += 16;
         w = (uint8_t *)(((uintptr_t)w + 15) & ~(uintptr_t)15);
+        totals_dev = (uint64_t *)w;       w += 32;
         partials = (uint64_t *)w;
     }
     a.tags = in.tags;
@@ -528,25 +567,26 @@ int serialize_outlines(gudni_ctx *ctx, const SerIn &in, const SerOut &out, SerCo
     a.ooff = in.ooff;
     a.pairs = in.pairs;
     a.n_shapes = n;
+    a.n_outlines = in.n_outlines;
+    a.n_pairs = in.n_pairs;
+    if (!out.curves) a.cstart = nullptr;   // no curve tracking: no curve scan
     a.fw = (float)in.width;
     a.fh = (float)in.height;
     a.subs = in.subs;
     a.n_subs = in.n_subs;
     a.n_uses = in.n_uses;
     a.n_grads = in.n_grads;
-    hipLaunchKernelGGL(ser::ser_reset, dim3(1), dim3(64), 0, st, a.status);
+    hipLaunchKernelGGL(ser::ser_knobs, dim3(ser::grid_for(in.n_pairs)), dim3(ser::kThreads), 0, st, a);
     hipLaunchKernelGGL(ser::ser_count, dim3(ser::grid_for(n)), dim3(ser::kThreads), 0, st, a);
     devscan::excl_scan(ser::KeepFlags{a.keep, n}, partials, a.kidx, st);
     devscan::excl_scan(ser::Units{a.units, n}, partials, a.ustart, st);
     if (out.curves) devscan::excl_scan(ser::Curves{a.units, a.strands, n}, partials, a.cstart, st);
+    hipLaunchKernelGGL(ser::ser_totals, dim3(1), dim3(1), 0, st, a, totals_dev);
     CHECK_HIP(ctx, hipGetLastError());
-    uint64_t totals[3] = {0, 0, 0};
-    uint32_t status = 0;
-    CHECK_HIP(ctx, hipMemcpyAsync(&totals[0], a.kidx + n, 8, hipMemcpyDeviceToHost, st));
-    CHECK_HIP(ctx, hipMemcpyAsync(&totals[1], a.ustart + n, 8, hipMemcpyDeviceToHost, st));
-    if (out.curves) CHECK_HIP(ctx, hipMemcpyAsync(&totals[2], a.cstart + n, 8, hipMemcpyDeviceToHost, st));
-    CHECK_HIP(ctx, hipMemcpyAsync(&status, a.status, 4, hipMemcpyDeviceToHost, st));
+    uint64_t totals[4] = {0, 0, 0, 0};
+    CHECK_HIP(ctx, hipMemcpyAsync(totals, totals_dev, sizeof(totals), hipMemcpyDeviceToHost, st));
     CHECK_HIP(ctx, hipStreamSynchronize(st));
+    const uint32_t status = (uint32_t)totals[3];
     if (status & ser::kErrSubstance)
         return set_error(ctx, GUDNI_ERR_ARG, "shape substance id outside the substance table");
     if (status & ser::kErrGradient)
@@ -580,17 +620,18 @@ int serialize_outlines_many(gudni_ctx *ctx, const SerIn *in, const SerOut *out, 
 {
     if (m <= 0) return GUDNI_OK;
     const hipStream_t st = ctx->stream;
-    // per scene: box 16n | units, kidx, ustart, cstart 8(n+1) | keep, strands 4n | status 16
-    auto ws_bytes = [](size_t n) {
-        return (16u * n + 8u * (4 * n + 3) + 4u * 2 * n + 16 + 255) & ~(size_t)255;
+    // per scene: box 16n | units, kidx, ustart, cstart 8(n+1) | keep, strands 4n | knobs 4p | status 16
+    auto ws_bytes = [](size_t n, size_t p) {
+        return (16u * n + 8u * (4 * n + 3) + 4u * 2 * n + 4u * p + 16 + 255) & ~(size_t)255;
     };
     std::vector<size_t> off((size_t)m);
     size_t total = 0;
-    int32_t most = 0;
+    int32_t most = 0, most_pairs = 0;
     for (int s = 0; s < m; ++s) {
         off[s] = total;
-        total += ws_bytes((size_t)in[s].n_shapes);
+        total += ws_bytes((size_t)in[s].n_shapes, (size_t)in[s].n_pairs);
         most = std::max(most, in[s].n_shapes);
+        most_pairs = std::max(most_pairs, in[s].n_pairs);
     }
     CHECK_HIP(ctx, ctx->ser_many_ws.ensure(total + 32u * (size_t)m));
     std::vector<ser::Args> args((size_t)m);
@@ -606,6 +647,7 @@ int serialize_outlines_many(gudni_ctx *ctx, const SerIn *in, const SerOut *out, 
         a.cstart = (uint64_t *)w;         w += 8u * (n + 1);
         a.keep = (uint32_t *)w;           w += 4u * n;
         a.strands = (uint32_t *)w;        w += 4u * n;
+        a.knob = (float *)w;              w += 4u * (size_t)in[s].n_pairs;
         a.status = (uint32_t *)w;
         if (!out[s].curves) a.cstart = nullptr;   // no curve tracking: no curve scan
         a.tags = in[s].tags;
@@ -613,6 +655,8 @@ int serialize_outlines_many(gudni_ctx *ctx, const SerIn *in, const SerOut *out, 
         a.ooff = in[s].ooff;
         a.pairs = in[s].pairs;
         a.n_shapes = in[s].n_shapes;
+        a.n_outlines = in[s].n_outlines;
+        a.n_pairs = in[s].n_pairs;
         a.fw = (float)in[s].width;
         a.fh = (float)in[s].height;
         a.subs = in[s].subs;
@@ -624,7 +668,8 @@ int serialize_outlines_many(gudni_ctx *ctx, const SerIn *in, const SerOut *out, 
     CHECK_HIP(ctx, upload(ctx, ctx->ser_many_args, args.data(), sizeof(ser::Args) * args.size()));
     const ser::Args *dargs = (const ser::Args *)ctx->ser_many_args.p;
     const int gx = std::min(64, ser::grid_for(most));
-    hipLaunchKernelGGL(ser::ser_reset_many, dim3(1), dim3(ser::kThreads), 0, st, dargs, m);
+    hipLaunchKernelGGL(ser::ser_knobs_many, dim3(std::min(64, ser::grid_for(most_pairs)), m), dim3(ser::kThreads), 0,
+                       st, dargs);
     hipLaunchKernelGGL(ser::ser_count_many, dim3(gx, m), dim3(ser::kThreads), 0, st, dargs);
     hipLaunchKernelGGL(ser::ser_scans_many, dim3(m), dim3(ser::kThreads), 0, st, dargs, totals_dev);
     CHECK_HIP(ctx, hipGetLastError());
@@ -712,6 +757,8 @@ int gudni_scene_upload_outlines(gudni_ctx *ctx, const gudni_outlines *o, const g
     in.ooff = (const int32_t *)ctx->ser_ooff.p;
     in.pairs = (const float *)ctx->ser_pairs.p;
     in.n_shapes = n;
+    in.n_outlines = n_outlines;
+    in.n_pairs = n_pairs;
     in.width = sc->width;
     in.height = sc->height;
     in.subs = (const float4 *)ctx->subs.p;
