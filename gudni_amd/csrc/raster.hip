@@ -321,26 +321,34 @@ int ensure_scratch(gudni_ctx *ctx)
 
 // How many waves (2^split, a power of two up to 64) run a unit's 64 columns.
 // A frame of few units leaves most of the chip idle and lasts as long as its
-// slowest unit, and a wave whose columns are tall is slow: its lanes' sweeps
-// diverge, so 64 columns take many times as long as one.  Splitting gives each
-// part a wave (with the slot's rings divided among fewer lanes, each longer,
-// so fewer units are left to the retry pass), at the price of listing the
-// unit's strands once per part.  That price is small where columns are tall
-// and most of the work where they are a row or two, so the number of parts is
-// held to rows / 4 per wave slot, at most 5, for columns of `rows` pixels on
-// average.  On 4096 slots (ms at split 0, 1, ... 6):
-//   641x479, 22 units of 218 rows      3.6 2.8 2.4 2.1 2.0 1.8 1.7   takes 6
-//   64x64, 4 units of 16 rows      .16 .11 .10 .093 .085 .082 .080   takes 6
-//   800x600, 367 units of 20 rows       29  18  13  10 8.3 7.3 6.7   takes 5
-//   1000x701, 536 units of 20 rows      13  11 7.7 5.7 4.3 3.4 4.0   takes 5
-//   768x768, 2 jobs of ~500, 9 rows     18  15  14  12 10. 9.6  11   takes 4
-//   512x512, 4096 units of 1 row        18  20  25  35  56  97 180   takes 0
-//   1920x1080, 8160 units of 4 rows    5.3 5.3 5.8 6.6 8.6  13  22   takes 0
-constexpr int kPartsPerSlot = 5;
-static int split_units(int n_work, double pixels, int slots, int capacity)
+// slowest unit, and a wave of crowded or tall columns is slow: its lanes'
+// sweeps diverge, so 64 columns take many times as long as one.  Splitting
+// gives each part a wave (with the slot's rings divided among fewer lanes,
+// each longer, so fewer units are left to the retry pass), at the price of
+// setting up the tile and listing its strands once per part.  That price is
+// the smaller the more shapes a tile has, and most of the work where columns
+// are a row or two.  So the parts per wave slot are held to (shapes per tile /
+// 40)^2, between 0.3 (a wave on an idle SIMD costs nothing) and 4.25, less for
+// columns under 8 rows.  On 4096 slots, us at split 0, 1, ... 6:
+//   641x479, 22 units of 218 rows, 100 shapes  2967 1969 1613 1403 1292 1224 1153  takes 6
+//   64x64, 4 units, 16 rows, 11 shapes         169 110 96 85 81 78 77               takes 6
+//   1000x701, 536 units, 20 rows, 100          9931 7618 5443 4231 3417 3087 3885   takes 5
+//   2000x2000, 260 units, 240 rows, 97         17497 10540 6798 5163 4233 4652 5650 takes 5
+//   1500x1200, 470 units, 60 rows, 40          2260 1529 1093 931 853 1060 1528     takes 3
+//   512x512, 256 units, 16 rows, 53            2965 2265 1971 1698 1550 1667 2079   takes 4
+//   500x400, 224 units, 14 rows, 14            748 541 448 424 551 615 655          takes 2
+//   1920x1080, 540 units, 60 rows, 5           555 337 387 567 643 792 1074         takes 1
+//   1920x1080, 2040 units, 16 rows, 12         350 494 549 628 800 1172 1899        takes 0
+//   512x512, 4096 units, 1 row, 740            13717 16375 21365 31647 52426 ...    takes 0
+//   1920x1080, 8160 units, 4 rows, 95          3795 3839 4454 5475 7894 ...         takes 0
+constexpr int kPartsPerSlot = 5;   // bound of the parts per slot, for the retry list
+static int split_units(int n_work, double pixels, double refs, int slots, int capacity)
 {
-    const double rows = n_work > 0 ? pixels / (64.0 * n_work) : 0.0;
-    const double parts = std::min((double)capacity, slots * std::min((double)kPartsPerSlot, 0.25 * rows));
+    if (n_work <= 0) return 0;
+    const double rows = pixels / (64.0 * n_work), shapes = 4.0 * refs / n_work;
+    const double crowd = shapes / 40.0;
+    const double fill = std::min(4.25, std::max(0.3, crowd * crowd)) * std::min(1.0, rows / 8.0);
+    const double parts = std::min((double)capacity, slots * fill);
     int split = 0;
     while (split < 6 && (double)n_work * (double)(2 << split) <= parts) ++split;
     return split;
@@ -438,8 +446,9 @@ static PassBuffers ctx_buffers(gudni_ctx *ctx)
                        ctx->slow_blocks, 256};
 }
 
-// pixels: what the launch covers, for the choice of the split.
-static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, double pixels)
+// pixels, refs: what the launch covers and how many shape references its
+// tiles hold, for the choice of the split.
+static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, double pixels, double refs)
 {
     uint32_t *ctl = b.ctl;
     hipLaunchKernelGGL(dev::reset_counters, dim3(1), dim3(64), 0, ctx->stream, ctl, dev::kCtlWords);
@@ -456,7 +465,7 @@ static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, dou
     f.shape_idx = b.fast_sidx;
     int slog = 0;
     while ((1 << slog) < ctx->spec.max_thresholds) ++slog;
-    f.split = split_units(f.n_work, pixels, 4 * b.fast_blocks, b.retry_capacity);
+    f.split = split_units(f.n_work, pixels, refs, 4 * b.fast_blocks, b.retry_capacity);
     f.slot_log2 = dev::kFastCapLog2 + 6;
     f.cap_log2 = std::min(dev::kFastCapLog2 + f.split, std::max(slog, dev::kFastCapLog2));
     const int fast_grid = std::max(1, std::min(b.fast_blocks, ((f.n_work << f.split) + 3) / 4));
@@ -476,9 +485,9 @@ static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, dou
     return GUDNI_OK;
 }
 
-static int launch_passes(gudni_ctx *ctx, dev::Frame f, double pixels)
+static int launch_passes(gudni_ctx *ctx, dev::Frame f, double pixels, double refs)
 {
-    return launch_passes(ctx, f, ctx_buffers(ctx), pixels);
+    return launch_passes(ctx, f, ctx_buffers(ctx), pixels, refs);
 }
 
 int read_status(gudni_ctx *ctx)
@@ -643,7 +652,12 @@ int validate_job(gudni_ctx *ctx, const CommonView &cv, const ShapeRec *shapes,
 // launches): 250^2, 120 shapes, 16-px tiles (256 cells) 130 / 569; 640^2, 300,
 // 256 px (16) 108 / 825; 512^2, 1,000, 32 px (256) 344 / 675; 800^2, 3,000,
 // 256 px (16) 529 / 823; 1920^2, 1,000, 64 px (1,024) 764 / 963; beyond the
-// line 512^2, 2,000, 16 px (1,024) 1,047 / 685.
+// line 512^2, 2,000, 16 px (1,024) 1,047 / 685.  Large shapes reach most
+// tiles of a deep tree (580 scribbles on 102x462: 1.4M references, 15 ms in
+// one block): a build past its first capacity of pairs gives up and goes to
+// the launches, and so does the next scene of a context whose last one had
+// that many.
+constexpr int32_t kBlockPairs = 1 << 16;
 static bool one_block_scene(int64_t shapes, int64_t cells)
 {
     return shapes <= 4096 && cells <= 1024 && shapes * cells <= (1 << 20);
@@ -653,20 +667,23 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
 {
     const int side = ceil_log2(std::max(in.width, in.height)) -
                      ceil_log2(in.max_tile_size > 0 ? in.max_tile_size : ctx->spec.max_tile_size);
-    if (one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side))) {
+    if (ctx->bin_last_pairs <= kBlockPairs &&
+        one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side))) {
         if (ctx->timing) {
             for (hipEvent_t &e : ctx->bin_ev)
                 if (!e) CHECK_HIP(ctx, hipEventCreate(&e));
             CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[0], ctx->stream));
         }
-        const int rc = bin_scenes(ctx, &in, &out, &cnt, 1);
-        if (rc) return rc;
-        if (ctx->timing) {
-            CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[1], ctx->stream));
-            CHECK_HIP(ctx, hipEventSynchronize(ctx->bin_ev[1]));
-            CHECK_HIP(ctx, hipEventElapsedTime(&ctx->last_bin_ms, ctx->bin_ev[0], ctx->bin_ev[1]));
+        const int rc = bin_scenes(ctx, &in, &out, &cnt, 1, kBlockPairs);
+        if (rc < 0) return rc;
+        if (rc == GUDNI_OK) {
+            if (ctx->timing) {
+                CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[1], ctx->stream));
+                CHECK_HIP(ctx, hipEventSynchronize(ctx->bin_ev[1]));
+                CHECK_HIP(ctx, hipEventElapsedTime(&ctx->last_bin_ms, ctx->bin_ev[0], ctx->bin_ev[1]));
+            }
+            return GUDNI_OK;
         }
-        return GUDNI_OK;
     }
     binning::Params bp;
     bp.n_shapes = in.n_shapes;
@@ -728,10 +745,11 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
     cnt.n_tiles = (int32_t)status[1];
     cnt.n_refs = (int32_t)status[2];
     cnt.n_work = (int32_t)status[3];
+    ctx->bin_last_pairs = (int32_t)status[5];
     return GUDNI_OK;
 }
 
-int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n)
+int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n, int32_t give_up_pairs)
 {
     if (n <= 0) return GUDNI_OK;
     std::vector<binning::Params> params((size_t)n);
@@ -758,6 +776,7 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
         // count per tile, and tiles never outnumber nodes
         cap_pairs[s] = (int32_t)std::max<int64_t>(
             std::min<int64_t>(std::max<int64_t>(1 << 14, 8 * (int64_t)bp.n_shapes), 1 << 28), cap_nodes[s]);
+        if (give_up_pairs > 0) cap_pairs[s] = std::max(give_up_pairs, cap_nodes[s]);
     }
     std::vector<int> todo((size_t)n);
     for (int s = 0; s < n; ++s) todo[s] = s;
@@ -806,6 +825,8 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
                 cnt[s].n_tiles = (int32_t)st[1];
                 cnt[s].n_refs = (int32_t)st[2];
                 cnt[s].n_work = (int32_t)st[3];
+            } else if (st[0] == 1 && give_up_pairs > 0) {
+                return 1;
             } else if (st[0] == 1) {
                 // grow only what ran out; fail once it is at its clamp
                 const bool over_nodes = (st[6] & 1u) != 0, over_pairs = (st[6] & 2u) != 0;
@@ -1113,7 +1134,7 @@ static int run_job(gudni_ctx *ctx, const void *shapes, int32_t n_shapes, const v
         pixels += std::max(0.0, std::min(w, r.box[2]) - (double)r.box[0]) *
                   std::max(0.0, std::min(h, r.box[3]) - (double)r.box[1]);
     }
-    rc = launch_passes(ctx, f, pixels);
+    rc = launch_passes(ctx, f, pixels, n_shapes);
     if (rc) return rc;
     rc = read_status(ctx);
     if (rc) return rc;
@@ -1201,6 +1222,7 @@ int gudni_frame_upload(gudni_ctx *ctx, const gudni_jobs *jobs, int32_t width, in
     ctx->frame_h = height;
     ctx->frame_n_work = (int32_t)work.size();
     ctx->frame_n_tiles = v.n_tiles;
+    ctx->frame_n_refs = v.n_refs;
     ctx->frame_index = frame;
     ctx->frame_sort_bits = jobs->j.sort_radix_bits;
     std::memcpy(ctx->background, background, sizeof(ctx->background));
@@ -1232,7 +1254,7 @@ int gudni_frame_render(gudni_ctx *ctx, uint32_t *out_dev, float *out_f32_dev)
         CHECK_HIP(ctx, hipEventRecord(ctx->ev[0], ctx->stream));
     }
     ctx->timed_render = ctx->timing;
-    int rc = launch_passes(ctx, f, (double)ctx->frame_w * ctx->frame_h);
+    int rc = launch_passes(ctx, f, (double)ctx->frame_w * ctx->frame_h, ctx->frame_n_refs);
     if (rc) return rc;
     if (ctx->timing) CHECK_HIP(ctx, hipEventRecord(ctx->ev[2], ctx->stream));
     return GUDNI_OK;
@@ -1279,7 +1301,7 @@ int gudni_frame_render_static(gudni_ctx *ctx, uint32_t *out_dev, float *out_f32_
                         reinterpret_cast<float4 *>(base + kOffSlowThr),
                         reinterpret_cast<uint32_t *>(base + kOffSlowHdr),
                         reinterpret_cast<int32_t *>(base + kOffSlowSidx), 1, 64};
-    return launch_passes(ctx, f, b, (double)ctx->frame_w * ctx->frame_h);
+    return launch_passes(ctx, f, b, (double)ctx->frame_w * ctx->frame_h, ctx->frame_n_refs);
 }
 
 int gudni_frame_check(gudni_ctx *ctx)
@@ -1351,6 +1373,7 @@ int gudni_scene_bin(gudni_ctx *ctx)
     ctx->frame_h = ctx->scene_h;
     ctx->frame_n_tiles = (int32_t)status[1];
     ctx->scene_n_refs = (int32_t)status[2];
+    ctx->frame_n_refs = (int32_t)status[2];
     ctx->frame_n_work = (int32_t)status[3];
     ctx->frame_index = 0;
     ctx->frame_sort_bits = ctx->spec.sort_radix_bits;
@@ -1459,6 +1482,7 @@ struct gudni_batch {
     std::vector<int32_t> width, height;
     std::vector<int32_t> work_begin, work_count;
     int32_t n_work = 0;
+    size_t n_refs = 0;         // shape references of all scenes
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint64_t captured_gen = 0;     // ctx->scratch_gen the graph was captured with
@@ -1555,6 +1579,7 @@ int gudni_batch_upload(gudni_ctx *ctx, int32_t n_scenes, const gudni_batch_scene
     b->n_scenes = n_scenes;
     b->device = ctx->device;
     b->n_work = (int32_t)work.size();
+    b->n_refs = refs.size();
     b->frame_off = frame_off;
     b->work_begin = wbegin;
     b->work_count = wcount;
@@ -1782,6 +1807,7 @@ int gudni_batch_upload_outlines(gudni_ctx *ctx, int32_t n_scenes, const gudni_ou
         if (e == hipSuccess && !d->p) e = d->ensure(16);
     if (e != hipSuccess) return hip_fail(e);
     b->n_work = (int32_t)(work_used / 4);
+    b->n_refs = refs_used / 16;
     {
         std::vector<TileRec> th(tiles_used / 32);
         std::vector<int32_t> ts(tiles_used / 32);
@@ -1846,7 +1872,7 @@ static int batch_launch(gudni_ctx *ctx, gudni_batch *b)
     CHECK_HIP(ctx, hipGetLastError());
     double pixels = 0.0;
     for (int32_t s = 0; s < b->n_scenes; ++s) pixels += (double)b->width[s] * b->height[s];
-    return launch_passes(ctx, batch_frame(ctx, b), pixels);
+    return launch_passes(ctx, batch_frame(ctx, b), pixels, (double)b->n_refs);
 }
 
 int gudni_batch_render(gudni_ctx *ctx, gudni_batch *b, int use_graph)
@@ -1909,7 +1935,8 @@ int gudni_batch_render_scene(gudni_ctx *ctx, gudni_batch *b, int32_t scene)
     f.work = (const uint32_t *)b->work.p + b->work_begin[scene];
     f.n_work = b->work_count[scene];
     f.scene_done = nullptr;
-    return launch_passes(ctx, f, (double)b->width[scene] * b->height[scene]);
+    return launch_passes(ctx, f, (double)b->width[scene] * b->height[scene],
+                         (double)b->n_refs * f.n_work / std::max(1, b->n_work));
 }
 
 int gudni_batch_check(gudni_ctx *ctx, gudni_batch *b, float *latency_ms)
