@@ -392,7 +392,8 @@ __device__ __forceinline__ void generate_o(const Frame &f, const AdjDesc &d, Que
     uint32_t n_orig = 0;
     uint64_t c0 = 0, c1 = 0;
     bool any_nonzero = false;   // nonzero-fill shapes are refused
-    walk_strands<kCompact>(f, s, q, c, active, lane, span0, span1, sidx, tt->strands, shape_bits, stack0, stack1,
+    walk_strands<kCompact>(f, s, q, c, active, lane, span0, span1, sidx, tt->strands, columns_log2((int)(span1 - span0) - 2), shape_bits,
+                           stack0, stack1,
                            c0, c1, any_nonzero,
                            [&](uint32_t place, uint32_t meta, uint32_t bit, bool &added, bool &enclosed) {
                                const GUDNI_CONST uint8_t *strand = ro(s.geo) + 16ull * place;

@@ -436,6 +436,7 @@ constexpr uint32_t kStrandNonzero = 1u << 22, kStrandReversed = 1u << 23, kStran
 struct StrandList {
     float4 box[kStrands];
     uint2 ref[kStrands];
+    uint32_t rows[32 * 8];   // rows of 32 of them in a wave's columns, at most 8 (pack_rows)
 };
 
 // Per-wave LDS table of a compact tile's shapes by tile-local index: tag,
@@ -490,32 +491,57 @@ __device__ __forceinline__ bool curve_bounds(const Trav &t, float x0, float x1, 
     return d0 > 1e-3f && d1 > 1e-3f;
 }
 
-// Whether a strand that covers the column passes wholly above its segment
-// (-1), wholly below (1) or may meet it (0).  spawn's lines run between points
-// of the curve under the left border, of the one under the right border, and
-// from one curve to the other.  A border's y is a chord's, and a flat chord
-// lies within 0.25 (in x plus y) of its curve; so all of them lie outside the
-// segment where both curves do, over the column widened by half a pixel, by
-// the margin: 2 pixels and 1/256 of the curves' extent.
-__device__ __forceinline__ int strand_side(const SceneDesc &s, uint2 ref, float dx, float dy, float height)
+// Bounds (lo, hi), with their margin, on the y of a strand that covers the
+// column at dx, relative to dy; false where it has none.  spawn's lines run
+// between points of the curve under the left border, of the one under the
+// right border, and from one curve to the other.  A border's y is a chord's,
+// and a flat chord lies within 0.25 (in x plus y) of its curve; so all of them
+// lie within the bounds of both curves over the column widened by half a
+// pixel, and the margin: 2 pixels and 1/256 of the curves' extent.
+__device__ __forceinline__ bool strand_bounds(const SceneDesc &s, uint2 ref, float dx, float dy, float &lo, float &hi)
 {
-    if (ref.y & kStrandFar) return 0;
+    if (ref.y & kStrandFar) return false;
     const GUDNI_CONST uint8_t *strand = ro(s.geo) + 16ull * ref.x;
     Trav l = strand_view(strand, dx, dy), r = l;
     l.xpos = cl_max(0.0f, l.left.x);
     r.xpos = cl_min(1.0f, l.right.x);
     search_pair(l, r, strand + 32, ((int)(ref.y & 0xFFFFu) - 4) / 2, dx, dy);
-    float lo = FLT_MAX, hi = -FLT_MAX;
+    lo = FLT_MAX;
+    hi = -FLT_MAX;
     bool known = curve_bounds(l, fmaxf(l.left.x, -0.5f), fminf(1.5f, l.right.x), lo, hi);
     float extent = (l.right.x - l.left.x) + fabsf(l.ctl.y - l.left.y) + fabsf(l.right.y - l.ctl.y);
     if (l.index != r.index) {
         known = curve_bounds(r, fmaxf(r.left.x, -0.5f), fminf(1.5f, r.right.x), lo, hi) && known;
         extent = fmaxf(extent, (r.right.x - r.left.x) + fabsf(r.ctl.y - r.left.y) + fabsf(r.right.y - r.ctl.y));
     }
-    if (!known) return 0;
     const float margin = 2.0f + extent * (1.0f / 256.0f);
-    return hi <= -margin ? -1 : (lo >= height + margin ? 1 : 0);
+    lo -= margin;
+    hi += margin;
+    return known;
 }
+
+// Whether a strand that covers the column passes wholly above its segment
+// (-1), wholly below (1) or may meet it (0).
+__device__ __forceinline__ int strand_side(const SceneDesc &s, uint2 ref, float dx, float dy, float height)
+{
+    float lo, hi;
+    if (!strand_bounds(s, ref, dx, dy, lo, hi)) return 0;
+    return hi <= 0.0f ? -1 : (lo >= height ? 1 : 0);
+}
+
+// Rows [lo, hi) as 15 and 16 bits (rounded outwards, held to +-kRowMax, which
+// the segments' rows stay below), and whether the strand covers the column's
+// left border.
+constexpr float kRowMax = 16000.0f;
+__device__ __forceinline__ uint32_t pack_rows(float lo, float hi, bool border)
+{
+    const int a = (int)floorf(fminf(fmaxf(lo, -kRowMax), kRowMax)), b = (int)ceilf(fminf(fmaxf(hi, -kRowMax), kRowMax));
+    return ((uint32_t)b << 16) | (((uint32_t)a & 0x7FFFu) << 1) | (border ? 1u : 0u);
+}
+__device__ __forceinline__ int rows_lo(uint32_t w) { return (int)(w << 16) >> 17; }
+__device__ __forceinline__ int rows_hi(uint32_t w) { return (int)w >> 16; }
+// log2 of a wave's columns (a power of two) where they are at most 8, else -1.
+__device__ __forceinline__ int columns_log2(int n) { return n <= 8 ? __ffs(n) - 1 : -1; }
 
 // buildThresholdArray (Kernels.cl:1540-1595): every column of the wave takes
 // the strands of its tile's shapes in order and emits their thresholds.
@@ -525,7 +551,9 @@ __device__ __forceinline__ int strand_side(const SceneDesc &s, uint2 ref, float 
 // marks the strands that cross its own segment and runs only those, one a
 // step, so a step serves a different strand in every lane and there are as
 // many steps as the busiest lane has crossing strands (walking strand by
-// strand, the wave ran every strand that crossed any of its 64 columns).
+// strand, the wave ran every strand that crossed any of its 64 columns).  A
+// wave of at most 8 columns bounds each strand once a column, as many at a
+// time as fill its lanes, for all the column's segments; wider ones a lane.
 // What the other strands do to a column follows from their extents:
 //  * left of or right of the column (the reference's own range test): nothing;
 //  * wholly below the segment, by a pixel or more: no threshold, and none that
@@ -555,7 +583,7 @@ __device__ __forceinline__ int strand_side(const SceneDesc &s, uint2 ref, float 
 template <bool kCompact, class Emit>
 __device__ __forceinline__ void walk_strands(const Frame &f, const SceneDesc &s, const Queue &q, const Column &c,
                                              bool active, int lane, float span0, float span1, int32_t *sidx,
-                                             StrandList &list, uint32_t &shape_bits, uint64_t &stack0,
+                                             StrandList &list, int cols_log2, uint32_t &shape_bits, uint64_t &stack0,
                                              uint64_t &stack1, uint64_t &contrib0, uint64_t &contrib1,
                                              bool &any_nonzero, Emit &&emit)
 {
@@ -563,6 +591,12 @@ __device__ __forceinline__ void walk_strands(const Frame &f, const SceneDesc &s,
     const uint32_t max_shapes = (uint32_t)f.max_shapes;
     const int num_shapes = (int)__builtin_amdgcn_readfirstlane(c.num_shapes);
     const int shape_start = (int)__builtin_amdgcn_readfirstlane(c.shape_start);
+    float highest = active ? dy : FLT_MAX;
+    for (int o = 32; o > 0; o >>= 1) highest = fminf(highest, __shfl_xor(highest, o));
+    const float ux = span0 + 1.0f;
+    const int my_col = (int)(dx - ux), my_row = (int)(dy - highest), my_end = my_row + c.int_height;
+    if (__any(active && (float)my_end >= kRowMax)) cols_log2 = -1;
+    const int cmask = (1 << (cols_log2 & 3)) - 1;
     const float below = dy + c.float_height + 1.0f, above = dy - 1.0f;
     float lowest = active ? below : -FLT_MAX;   // nothing below it reaches the wave
     for (int o = 32; o > 0; o >>= 1) lowest = fmaxf(lowest, __shfl_xor(lowest, o));
@@ -666,37 +700,67 @@ __device__ __forceinline__ void walk_strands(const Frame &f, const SceneDesc &s,
             wave_sync();
             uint32_t todo[kStrands / 32];   // strands that this lane runs
 #pragma unroll
-            for (int g = 0; g < kStrands / 32; ++g) {
-                uint32_t m = 0;
-                const int e0 = 32 * g, e1 = min(e0 + 32, (int)n);
-                for (int e = e0; e < e1; ++e) {
-                    const float4 b = list.box[e];
-                    const uint32_t meta = __builtin_amdgcn_readfirstlane(list.ref[e].y);
-                    const float lx = b.x - dx;
-                    const bool in = lx <= 1.0f && b.y - dx > 0.0f;
-                    const bool over = b.w <= above && !(meta & kStrandNonzero);
-                    if (in && !over && !(b.z >= below)) m |= 1u << (e - e0);
-                    if (in && over && lx <= 0.0f) enc ^= 1ull << ((meta >> 16) & 63u);
-                }
-                todo[g] = alive ? m : 0u;
-            }
-            // of those, the ones whose curves come near the segment in this
-            // very column
-#pragma unroll
-            for (int g = 0; g < kStrands / 32; ++g) {
-                uint32_t m = todo[g], run = 0;
-                while (__any(m != 0u)) {
-                    if (m) {
-                        const uint32_t bit = m & (0u - m);
-                        m ^= bit;
-                        const int e = 32 * g + __ffs((int)bit) - 1;
-                        const uint2 ref = list.ref[e];
-                        const int side = strand_side(s, ref, dx, dy, c.float_height);
-                        if (side == 0 || (side < 0 && (ref.y & kStrandNonzero))) run |= bit;
-                        else if (side < 0 && list.box[e].x - dx <= 0.0f) enc ^= 1ull << ((ref.y >> 16) & 63u);
+            for (int g = 0; g < kStrands / 32; ++g) todo[g] = 0u;
+            // rolled, the word chosen by selects: the body is long
+#pragma unroll 1
+            for (int e0 = 0; e0 < (int)n; e0 += 32) {
+                uint32_t run = 0;
+                const int e1 = min(e0 + 32, (int)n);
+                if (cols_log2 >= 0) {
+                    wave_sync();
+                    for (int i = lane; i < (e1 - e0) << cols_log2; i += kWave) {
+                        const float4 b = list.box[e0 + (i >> cols_log2)];
+                        const uint2 ref = list.ref[e0 + (i >> cols_log2)];
+                        const float cx = ux + (float)(i & cmask), cy = highest;
+                        const float lx = b.x - cx;
+                        uint32_t rows = pack_rows(kRowMax, kRowMax, false);   // does not cover the column
+                        if (lx <= 1.0f && b.y - cx > 0.0f) {
+                            float lo, hi;
+                            if (!strand_bounds(s, ref, cx, cy, lo, hi)) {
+                                lo = b.z - cy - 1.0f;
+                                hi = b.w - cy + 1.0f;
+                            }
+                            rows = pack_rows(lo, hi, lx <= 0.0f);
+                        }
+                        list.rows[i] = rows;
+                    }
+                    wave_sync();
+                    for (int e = e0; e < e1; ++e) {
+                        const uint32_t rows = list.rows[((e - e0) << cols_log2) + (my_col & cmask)];
+                        const uint32_t meta = __builtin_amdgcn_readfirstlane(list.ref[e].y);
+                        const bool over = rows_hi(rows) <= my_row && !(meta & kStrandNonzero);
+                        if (!over && rows_lo(rows) < my_end) run |= 1u << (e - e0);
+                        if (over && (rows & 1u)) enc ^= 1ull << ((meta >> 16) & 63u);
+                    }
+                    run = alive ? run : 0u;
+                } else {
+                    uint32_t m = 0;
+                    for (int e = e0; e < e1; ++e) {
+                        const float4 b = list.box[e];
+                        const uint32_t meta = __builtin_amdgcn_readfirstlane(list.ref[e].y);
+                        const float lx = b.x - dx;
+                        const bool in = lx <= 1.0f && b.y - dx > 0.0f;
+                        const bool over = b.w <= above && !(meta & kStrandNonzero);
+                        if (in && !over && !(b.z >= below)) m |= 1u << (e - e0);
+                        if (in && over && lx <= 0.0f) enc ^= 1ull << ((meta >> 16) & 63u);
+                    }
+                    m = alive ? m : 0u;
+                    // of those, the ones whose curves come near the segment in
+                    // this very column
+                    while (__any(m != 0u)) {
+                        if (m) {
+                            const uint32_t bit = m & (0u - m);
+                            m ^= bit;
+                            const int e = e0 + __ffs((int)bit) - 1;
+                            const uint2 ref = list.ref[e];
+                            const int side = strand_side(s, ref, dx, dy, c.float_height);
+                            if (side == 0 || (side < 0 && (ref.y & kStrandNonzero))) run |= bit;
+                            else if (side < 0 && list.box[e].x - dx <= 0.0f) enc ^= 1ull << ((ref.y >> 16) & 63u);
+                        }
                     }
                 }
-                todo[g] = run;
+#pragma unroll
+                for (int g = 0; g < kStrands / 32; ++g) todo[g] = e0 == 32 * g ? run : todo[g];
             }
             for (;;) {
                 int e = -1;
@@ -755,13 +819,13 @@ __device__ __forceinline__ void walk_strands(const Frame &f, const SceneDesc &s,
 
 template <bool kCompact>
 __device__ __forceinline__ void generate(const Frame &f, const SceneDesc &s, Queue &q, const Column &c, bool active, int lane,
-                         float span0, float span1, int32_t *sidx, TileTable *tt,
+                         float span0, float span1, int32_t *sidx, TileTable *tt, int cols_log2,
                          uint32_t &shape_bits, uint64_t &stack0, uint64_t &stack1,
                          uint64_t &contrib0, uint64_t &contrib1, bool &any_nonzero)
 {
     const float dx = (float)c.dx, dy = (float)c.dy;
-    walk_strands<kCompact>(f, s, q, c, active, lane, span0, span1, sidx, tt->strands, shape_bits, stack0, stack1,
-                           contrib0, contrib1, any_nonzero,
+    walk_strands<kCompact>(f, s, q, c, active, lane, span0, span1, sidx, tt->strands, cols_log2, shape_bits, stack0,
+                           stack1, contrib0, contrib1, any_nonzero,
                            [&](uint32_t place, uint32_t meta, uint32_t bit, bool &added, bool &enclosed) {
                                const GUDNI_CONST uint8_t *strand = ro(s.geo) + 16ull * place;
                                Trav l = strand_view(strand, dx, dy), r = l;
@@ -1681,7 +1745,8 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
         const int uw = unit_width(t.hdepth, f.compute_depth), lanes = kWave >> f.split;
         if (lanes < uw) x0 += (part * lanes) & (uw - 1);
         const int x1 = x0 + min(uw, lanes);
-        generate<kCompact>(f, s, q, c, active, lane, (float)x0 - 1.0f, (float)x1 + 1.0f, sidx, tt, bits,
+        generate<kCompact>(f, s, q, c, active, lane, (float)x0 - 1.0f, (float)x1 + 1.0f, sidx, tt,
+                           columns_log2(x1 - x0), bits,
                            s0, s1, c0, c1, any_nonzero);
     }
     const bool ok = active && !q.spilled && !q.overflow;
