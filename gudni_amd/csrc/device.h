@@ -497,7 +497,7 @@ __device__ __forceinline__ bool curve_bounds(const Trav &t, float x0, float x1, 
 // right border, and from one curve to the other.  A border's y is a chord's,
 // and a flat chord lies within 0.25 (in x plus y) of its curve; so all of them
 // lie within the bounds of both curves over the column widened by half a
-// pixel, and the margin: 2 pixels and 1/256 of the curves' extent.
+// pixel, and the margin: a pixel and 1/256 of the curves' extent.
 __device__ __forceinline__ bool strand_bounds(const SceneDesc &s, uint2 ref, float dx, float dy, float &lo, float &hi)
 {
     if (ref.y & kStrandFar) return false;
@@ -514,7 +514,7 @@ __device__ __forceinline__ bool strand_bounds(const SceneDesc &s, uint2 ref, flo
         known = curve_bounds(r, fmaxf(r.left.x, -0.5f), fminf(1.5f, r.right.x), lo, hi) && known;
         extent = fmaxf(extent, (r.right.x - r.left.x) + fabsf(r.ctl.y - r.left.y) + fabsf(r.right.y - r.ctl.y));
     }
-    const float margin = 2.0f + extent * (1.0f / 256.0f);
+    const float margin = 1.0f + extent * (1.0f / 256.0f);
     lo -= margin;
     hi += margin;
     return known;
@@ -646,33 +646,43 @@ __device__ __forceinline__ void walk_strands(const Frame &f, const SceneDesc &s,
         for (uint32_t w0 = 0; w0 < total;) {
             const uint32_t w1 = min(total, w0 + (uint32_t)kStrands - n);
             wave_sync();
-            while (listed < ns && start + listed < w1) {
+            if (listed < ns && start + listed < w1) {
+                // the next strand's head and first curve come with this
+                // one's curves
                 const GUDNI_CONST uint8_t *p = ro(s.geo) + 16ull * place;
-                const float4 h = ld4(p), first = ld4(p + 16);
-                const uint32_t head = __float_as_uint(h.x), size = head & 0xFFFFu;
-                float lo = h.w, hi = h.w, far = fmaxf(fabsf(h.z), fabsf(h.w));
-                bool nan = !(h.z == h.z) || !(h.w == h.w);
-                const int m = (int)size / 2;   // float4s of the strand
-                float4 v = first;
-                for (int i = 1;;) {
-                    lo = fminf(lo, fminf(v.y, v.w));
-                    hi = fmaxf(hi, fmaxf(v.y, v.w));
-                    far = fmaxf(far, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-                    nan = nan || !(v.x == v.x) || !(v.y == v.y) || !(v.z == v.z) || !(v.w == v.w);
-                    if (++i >= m) break;
-                    v = ld4(p + 16 * i);
+                float4 h = ld4(p);
+                for (bool more = true; more;) {
+                    const uint32_t head = __float_as_uint(h.x), size = head & 0xFFFFu;
+                    const int m = (int)size / 2;   // float4s of the strand
+                    const uint32_t e = n + start + listed - w0;
+                    ++listed;
+                    more = listed < ns && start + listed < w1;
+                    const GUDNI_CONST uint8_t *next = p + 16 * m;
+                    const float4 first = ld4(p + 16), nh = ld4(more ? next : p);
+                    float4 v = m > 2 ? ld4(p + 32) : first;
+                    float lo = fminf(h.w, fminf(first.y, first.w)), hi = fmaxf(h.w, fmaxf(first.y, first.w));
+                    // the largest magnitude, as bits: those of a NaN exceed all
+                    auto mag = [](float x) { return __float_as_uint(x) & 0x7FFFFFFFu; };
+                    auto mag4 = [&](float4 x) { return max(max(mag(x.x), mag(x.y)), max(mag(x.z), mag(x.w))); };
+                    uint32_t far = max(max(mag(h.z), mag(h.w)), mag4(first));
+                    for (int i = 2; i < m;) {
+                        lo = fminf(lo, fminf(v.y, v.w));
+                        hi = fmaxf(hi, fmaxf(v.y, v.w));
+                        far = max(far, mag4(v));
+                        if (++i < m) v = ld4(p + 16 * i);
+                    }
+                    const bool wild = far >= __float_as_uint(1048576.0f);
+                    if (wild) {
+                        lo = shape_top;
+                        hi = INFINITY;
+                    }
+                    list.box[e] = make_float4(first.x, h.z, lo, hi);
+                    list.ref[e] = make_uint2(place, size | ((uint32_t)lane << 16) | rule | (wild ? kStrandFar : 0u) |
+                                                        (rule && ((head >> 16) & GUDNI_STRAND_REVERSED) ? kStrandReversed : 0u));
+                    place += size / 2;
+                    p = next;
+                    h = nh;
                 }
-                const bool wild = nan || far >= 1048576.0f;
-                if (wild) {
-                    lo = shape_top;
-                    hi = INFINITY;
-                }
-                const uint32_t e = n + start + listed - w0;
-                list.box[e] = make_float4(first.x, h.z, lo, hi);
-                list.ref[e] = make_uint2(place, size | ((uint32_t)lane << 16) | rule | (wild ? kStrandFar : 0u) |
-                                                    (rule && ((head >> 16) & GUDNI_STRAND_REVERSED) ? kStrandReversed : 0u));
-                place += size / 2;
-                ++listed;
             }
             wave_sync();
             // of these, the list keeps those that reach the wave's columns
