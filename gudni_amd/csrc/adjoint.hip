@@ -105,8 +105,13 @@ struct AdjFrame {
     float4 *q_cols;               // [slots][kStream][64]: the colours of each lane's first sections
 };
 
-// Section colours that a lane keeps from the forward sweep for the backward.
+// Section colours that a lane keeps from the forward sweep for the backward,
+// which also keeps the colours of its listed sections there, in the row of
+// each one's number among them.  That row's forward colour has been read (a
+// section is listed after it is swept), and no section that still waits in the
+// list has it (a list holds fewer sections than there are rows).
 constexpr int kStream = 256;
+static_assert(kSections < kStream && kStream <= 256, "a list entry names its row with 8 bits");
 
 enum Mode { kRecord = 0, kApply = 1 };
 
@@ -838,15 +843,13 @@ __device__ __forceinline__ uint32_t sweep_forward(const AdjDesc &d, Queue &q, co
 }
 
 // Backward sweep over the same sections.  A lane takes its sections' colours
-// from the forward's stream (past its kStream rows it evaluates them, and
-// keeps them in the row its section's number falls on) and adds the boundary
-// terms; the colour gradients, the bulk of the work, are listed and walked a
-// section a lane by the whole wave.  (Evaluating the colours again here, each
-// lane for itself, took half of this sweep.)  With both sweeps listed and
-// generation's strand choice the 1024^2, 2,000-shape step went from 5.5 to 3.8
-// ms, eight textured 512^2 scenes from 19.2 to 14.5 (3.3 and 12.7 with strands
-// bounded a column).  Every lane of the wave
-// calls it.
+// from the forward's stream (past its kStream rows it evaluates them) and adds
+// the boundary terms; the colour gradients, the bulk of the work, are listed
+// and walked a section a lane by the whole wave.  (Evaluating the colours again
+// here, each lane for itself, took half of this sweep.)  With both sweeps
+// listed and generation's strand choice the 1024^2, 2,000-shape step went from
+// 5.5 to 3.8 ms, eight textured 512^2 scenes from 19.2 to 14.5 (3.3 and 12.7
+// with strands bounded a column).  Every lane of the wave calls it.
 template <bool kCompact>
 __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc &d, Queue &q, const Column &c,
                                                    Stack st, const int32_t *sidx, TileTable *tt,
@@ -859,7 +862,9 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
     Sweep p;
     start_sweep(p, st);
     int guard = (int)kSectionGuard;
-    uint32_t status = 0, row = 0, seq = 0;
+    // sections swept and sections listed: seq numbers the forward's rows,
+    // listed the rows that hold listed sections' colours
+    uint32_t status = 0, row = 0, seq = 0, listed = 0;
     bool alive = ok && p.pixel_y <= c.float_height;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 G = alive ? d.gpix[(long long)c.dy * s.width + c.dx] : zero;
@@ -881,7 +886,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
         bool have = false;
         float area = 0.0f;
         uint64_t s0 = 0, s1 = 0;
-        const uint32_t at = (uint32_t)lane | (row << 6) | ((seq & (uint32_t)(kStream - 1)) << 24);
+        uint32_t at = 0;
         if (alive && (advance || !border)) {
             if (!((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y))) {
                 // the pixel's end; the span state starts afresh
@@ -932,13 +937,8 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                     p.sx0 = p.sx1;
                     p.sx1 = nx;
                     float4 col;
-                    if (seq < (uint32_t)kStream) {
-                        col = cols[seq * kWave];
-                    } else {
-                        col = determine_color<kCompact>(f, s, st, sidx, tt, c.dx, c.dy + (int)row);
-                        cols[(seq & (uint32_t)(kStream - 1)) * kWave] = col;
-                    }
-                    ++seq;
+                    if (seq < (uint32_t)kStream) col = cols[seq * kWave];
+                    else col = determine_color<kCompact>(f, s, st, sidx, tt, c.dx, c.dy + (int)row);
                     const float dy = p.sy1 - p.sy0;
                     area = (p.sx1 - p.sx0) * dy;
                     float et = 1.0f, eb = 1.0f;
@@ -972,6 +972,13 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                         }
                     }
                     have = G.x * area != 0.0f || G.y * area != 0.0f || G.z * area != 0.0f || G.w * area != 0.0f;
+                    if (have) {
+                        const uint32_t k = listed & (uint32_t)(kStream - 1);
+                        if (listed != seq || seq >= (uint32_t)kStream) cols[k * kWave] = col;
+                        at = (uint32_t)lane | (row << 6) | (k << 24);
+                        ++listed;
+                    }
+                    ++seq;
                     s0 = st.s0;
                     s1 = st.s1;
                     if (crossing) {
