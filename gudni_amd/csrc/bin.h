@@ -69,6 +69,7 @@ struct SceneJob {
     const ShapeRec *shapes;
     const float4 *bbox, *shape_bounds;
     Output out;
+    int32_t give_up;   // stop with status[0] = 1 as soon as the pairs are seen to outgrow cap_pairs
 };
 
 constexpr int kSceneBlockThreads = 512;

@@ -439,6 +439,27 @@ __global__ void __launch_bounds__(kThreads) bin_emit_work(Dev d, WorkFlags f, ui
     emit_work_body(d, f, work, gtid(), gstride());
 }
 
+// Whether the pairs of all levels will outgrow the capacity, after `level` has
+// been advanced: while the next nodes are forced to split or hold cap_shapes
+// shapes on average, a level's pairs grow as this one's did (a shape crosses
+// more cuts the smaller the nodes are, so this is low rather than high).  The
+// first two levels are not asked: their nodes are larger than most shapes.
+__device__ bool outgrows(const Dev &d, int level)
+{
+    if (level < 1 || level + 1 >= d.p.max_levels) return false;
+    const int4 lv = d.levels[level], nx = d.levels[level + 1];
+    if (lv.w == 0) return false;
+    const float grow = (float)nx.w / (float)lv.w;
+    float nodes = (float)nx.y, pairs = (float)nx.w, total = (float)(nx.z + nx.w);
+    const int forced = 2 * (d.p.canvas_depth - d.p.tile_depth), last = 2 * (d.p.canvas_depth - 3);
+    for (int l = level + 1; l < last && (l < forced || pairs >= nodes * (float)d.p.cap_shapes); ++l) {
+        nodes *= 2.0f;
+        pairs *= grow;
+        total += pairs;
+    }
+    return total > (float)d.cap_pairs;
+}
+
 // One scene per block: the steps of enqueue() in order, with block barriers
 // for the kernel boundaries and block scans for the device-wide ones.
 __global__ void __launch_bounds__(kSceneBlockThreads) bin_scene_block(const SceneJob *jobs)
@@ -473,7 +494,13 @@ __global__ void __launch_bounds__(kSceneBlockThreads) bin_scene_block(const Scen
         devscan::block_range_excl_scan(
             PairFlags{d.levels, d.node_meta, d.node_box, d.pair_shape, d.pair_node, j.bbox, l, 0, 0}, d.scan);
         __syncthreads();
-        if (t0 == 0) advance_body(d, l);
+        if (t0 == 0) {
+            advance_body(d, l);
+            if (j.give_up && !d.status[0] && outgrows(d, l)) {
+                d.status[6] = 2u;
+                d.status[0] = 1u;
+            }
+        }
         __syncthreads();
         children_body(d, l, t0, ts);
         __syncthreads();

@@ -83,7 +83,6 @@ struct gudni_ctx {
     int32_t scene_n_shapes = 0, scene_w = 0, scene_h = 0;
     float scene_bg[4] = {1, 1, 1, 1};
     int32_t bin_cap_pairs = 0, bin_cap_nodes = 0, scene_n_refs = 0;
-    int32_t bin_last_pairs = 0;   // pairs of the last tree built by the level launches
     bool scene_ready = false;
     hipEvent_t bin_ev[2] = {nullptr, nullptr};
     float last_bin_ms = 0;
@@ -182,8 +181,8 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
 // The same for n scenes at once, one block per scene (for scenes of a few
 // thousand shapes, where the per-level launches of bin_scene cost more than
 // the work): one launch and one synchronisation while the capacities hold.
-// give_up_pairs > 0: a scene of more (node, shape) pairs than that is not
-// built; returns 1 then.
+// give_up_pairs > 0: a scene that has or will have more (node, shape) pairs
+// than that is not built; returns 1 then.
 int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n, int32_t give_up_pairs = 0);
 // Bounds-checks shape records (and tiles) against the common buffers and
 // fills each shape's strand extent (xmin, ymin, xmax, ymax).

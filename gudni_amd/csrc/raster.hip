@@ -655,9 +655,11 @@ int validate_job(gudni_ctx *ctx, const CommonView &cv, const ShapeRec *shapes,
 // 256 px (16) 529 / 823; 1920^2, 1,000, 64 px (1,024) 764 / 963; beyond the
 // line 512^2, 2,000, 16 px (1,024) 1,047 / 685.  Large shapes reach most
 // tiles of a deep tree (580 scribbles on 102x462: 1.4M references, 15 ms in
-// one block): a build past its first capacity of pairs gives up and goes to
-// the launches, and so does the next scene of a context whose last one had
-// that many.
+// one block): a build that passes its first capacity of pairs, or is seen to
+// grow past it (outgrows), gives up and goes to the launches.  Every scene is
+// tried alike, whatever the context built before.  Giving up costs 40 us (1,000
+// scribbles on 512^2: 790 us in all, 742 by the launches alone; 1,100 where the
+// block filled its capacity first).
 constexpr int32_t kBlockPairs = 1 << 16;
 static bool one_block_scene(int64_t shapes, int64_t cells)
 {
@@ -668,8 +670,7 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
 {
     const int side = ceil_log2(std::max(in.width, in.height)) -
                      ceil_log2(in.max_tile_size > 0 ? in.max_tile_size : ctx->spec.max_tile_size);
-    if (ctx->bin_last_pairs <= kBlockPairs &&
-        one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side))) {
+    if (one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side))) {
         if (ctx->timing) {
             for (hipEvent_t &e : ctx->bin_ev)
                 if (!e) CHECK_HIP(ctx, hipEventCreate(&e));
@@ -746,7 +747,6 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
     cnt.n_tiles = (int32_t)status[1];
     cnt.n_refs = (int32_t)status[2];
     cnt.n_work = (int32_t)status[3];
-    ctx->bin_last_pairs = (int32_t)status[5];
     return GUDNI_OK;
 }
 
@@ -809,6 +809,7 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
             j.shapes = in[s].shapes;
             j.bbox = in[s].bbox;
             j.shape_bounds = in[s].bounds;
+            j.give_up = give_up_pairs > 0 ? 1 : 0;
             j.out = binning::Output{(TileRec *)o.tiles->p, (int32_t *)o.tile_job->p, (ShapeRec *)o.refs->p,
                                     (float4 *)o.ref_bounds->p, (uint32_t *)o.work->p};
         }
