@@ -1894,7 +1894,7 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
             atomicAdd(f.stage_cycles + 0, (unsigned long long)(t1 - t0));
             atomicAdd(f.stage_cycles + 1, (unsigned long long)(t2 - t1));
             atomicAdd(f.stage_cycles + 2, (unsigned long long)(t3 - t2));
-            atomicAdd(f.stage_cycles + 3, 1ull);
+            if (part == 0) atomicAdd(f.stage_cycles + 3, 1ull);   // a unit counts once, however many waves run it
         }
     }
 }
