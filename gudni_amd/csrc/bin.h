@@ -37,7 +37,9 @@ struct Workspace {
     int32_t *node_child = nullptr, *node_leaves = nullptr, *node_refs = nullptr;
     int32_t *node_toff = nullptr, *node_roff = nullptr;    // cap_nodes
     int4 *levels = nullptr;        // per level: node begin, node count, pair begin, pair count
-    uint32_t *status = nullptr;    // [0] overflow [1] tiles [2] refs [3] work [4] nodes [5] pairs
+    // [0] overflow [1] tiles [2] refs [3] work [4] nodes [5] pairs [6] what
+    // overflowed [7] shapes of all work units (unit_weight)
+    uint32_t *status = nullptr;
 };
 
 size_t workspace_bytes(int32_t cap_pairs, int32_t cap_nodes, int32_t max_levels);

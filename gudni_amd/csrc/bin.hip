@@ -95,6 +95,8 @@ __device__ bool quarter_active(const TileRec &r, int qd, int cd, int width, int 
     return false;
 }
 
+// A tile's work units, and in the upper half their shapes (unit_weight; at most
+// 4 x 2^28).
 struct WorkFlags {
     const TileRec *tiles;
     const uint32_t *status;
@@ -107,7 +109,7 @@ struct WorkFlags {
         const TileRec r = tiles[t];
         uint64_t k = 0;
         for (int q = 0; q < quarters; ++q) k += quarter_active(r, q, cd, width, height) ? 1u : 0u;
-        return k;
+        return k | (unit_weight((uint32_t)k) * (uint64_t)(uint32_t)r.shape_count) << 32;
     }
 };
 
@@ -431,7 +433,10 @@ __device__ void emit_work_body(const Dev &d, WorkFlags f, uint32_t *work, int t0
         for (int q = 0; q < f.quarters; ++q)
             if (quarter_active(r, q, f.cd, f.width, f.height)) work[k++] = ((uint32_t)t << 2) | (uint32_t)q;
     }
-    if (t0 == 0) d.status[3] = (uint32_t)d.scan[n];
+    if (t0 == 0) {
+        d.status[3] = (uint32_t)d.scan[n];
+        d.status[7] = (uint32_t)(d.scan[n] >> 32);
+    }
 }
 
 __global__ void __launch_bounds__(kThreads) bin_emit_work(Dev d, WorkFlags f, uint32_t *work)

@@ -73,7 +73,8 @@ struct gudni_ctx {
     // library's static scratch after gudni_frame_render_static)
     uint32_t *status_word = nullptr;
     // uploaded frame (Level 2)
-    int32_t frame_w = 0, frame_h = 0, frame_n_work = 0, frame_n_tiles = 0, frame_n_refs = 0, frame_index = 0;
+    int32_t frame_w = 0, frame_h = 0, frame_n_work = 0, frame_n_tiles = 0, frame_index = 0;
+    double frame_unit_shapes = 0;    // shapes of all work units (unit_weight)
     int32_t frame_sort_bits = 0;  // sort radix of the spec the uploaded jobs were built with
     float background[4] = {1, 1, 1, 1};
     bool frame_ready = false;
@@ -176,6 +177,7 @@ struct BinOut {
 };
 struct BinCounts {
     int32_t n_tiles = 0, n_refs = 0, n_work = 0;
+    uint32_t unit_shapes = 0;      // shapes of all work units (unit_weight)
 };
 int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt);
 // The same for n scenes at once, one block per scene (for scenes of a few

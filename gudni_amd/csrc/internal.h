@@ -70,6 +70,13 @@ constexpr int unit_column(int hd, int cd, int q, int lane)
     const int seg = ((q / u.n_x) << u.sw_bits) | (lane >> u.cw_bits);
     return (seg << hd) | x;
 }
+
+// How often the shapes of a tile of k active work units count among the shapes
+// of all units, by which a launch chooses how many waves run a unit: once a
+// unit, and twice for a tile of one (an 8-pixel tile, whose shapes cross half
+// as many columns).
+constexpr uint32_t unit_weight(uint32_t k) { return k == 1u ? 2u : k; }
+
 // First column (tile-relative) and width of unit q's block.
 constexpr int unit_x0(int hd, int cd, int q) { return (q % unit_shape(hd, cd).n_x) << unit_shape(hd, cd).cw_bits; }
 constexpr int unit_width(int hd, int cd) { return 1 << unit_shape(hd, cd).cw_bits; }

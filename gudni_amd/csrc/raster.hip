@@ -213,6 +213,18 @@ void build_work(const gudni_spec &spec, const TileRec *tiles, int n_tiles, int w
     }
 }
 
+// The shapes of all work units together (unit_weight); a tile's units follow
+// each other in the list.
+static uint64_t unit_shapes(const TileRec *tiles, const std::vector<uint32_t> &work)
+{
+    uint64_t n = 0;
+    for (size_t i = 0, k; i < work.size(); i += k) {
+        for (k = 1; i + k < work.size() && work[i + k] >> 2 == work[i] >> 2;) ++k;
+        n += unit_weight((uint32_t)k) * (uint64_t)(uint32_t)tiles[work[i] >> 2].shape_count;
+    }
+    return n;
+}
+
 void order_longest_first(int threads_per_tile, const TileRec *tiles, const int32_t *tile_scene,
                          const uint32_t *work, int n, int parts, uint32_t *out)
 {
@@ -326,30 +338,44 @@ int ensure_scratch(gudni_ctx *ctx)
 // sweeps diverge, so 64 columns take many times as long as one.  Splitting
 // gives each part a wave (with the slot's rings divided among fewer lanes,
 // each longer, so fewer units are left to the retry pass), at the price of
-// setting up the tile and listing its strands once per part.  That price is
-// the smaller the more shapes a tile has, and most of the work where columns
-// are a row or two.  So the parts per wave slot are held to (shapes per tile /
-// 40)^2, between 0.3 (a wave on an idle SIMD costs nothing) and 4.25, less for
-// columns under 8 rows.  On 4096 slots, us at split 0, 1, ... 6:
-//   641x479, 22 units of 218 rows, 100 shapes  2967 1969 1613 1403 1292 1224 1153  takes 6
-//   64x64, 4 units, 16 rows, 11 shapes         169 110 96 85 81 78 77               takes 6
-//   1000x701, 536 units, 20 rows, 100          9931 7618 5443 4231 3417 3087 3885   takes 5
-//   2000x2000, 260 units, 240 rows, 97         17497 10540 6798 5163 4233 4652 5650 takes 5
-//   1500x1200, 470 units, 60 rows, 40          2260 1529 1093 931 853 1060 1528     takes 3
-//   512x512, 256 units, 16 rows, 53            2965 2265 1971 1698 1550 1667 2079   takes 4
-//   500x400, 224 units, 14 rows, 14            748 541 448 424 551 615 655          takes 2
-//   1920x1080, 540 units, 60 rows, 5           555 337 387 567 643 792 1074         takes 1
-//   1920x1080, 2040 units, 16 rows, 12         350 494 549 628 800 1172 1899        takes 0
-//   512x512, 4096 units, 1 row, 740            13717 16375 21365 31647 52426 ...    takes 0
-//   1920x1080, 8160 units, 4 rows, 95          3795 3839 4454 5475 7894 ...         takes 0
+// claiming the part, setting up its tile and listing the tile's strands once
+// more.  So the parts per wave slot are held to
+//   (shapes per unit / 34)^2, less for columns under 6 rows, where the listing
+//   is most of the work; at most 4.25, and less the taller columns over 30 rows
+//   are, down to 1.25 (a column of 100 rows lasts long enough by itself);
+//   at least 0.3 (a wave on an idle SIMD costs little), less for columns under
+//   8 rows, and less where a column's rows and shapes are so few that it costs
+//   no more than its claim.
+// Shapes are counted over the work units, not over all tiles: the tree covers a
+// square, and a shape beside the canvas is held by the tiles there, which have no
+// units (4000x37 of a 4000^2 scene in 32-px tiles: 19 shapes a unit, 694
+// references for each four units).  On 435 frames of 16^2 to 4096x1024 pixels
+// and 8- to 256-px tiles the split taken costs 2.6% more than the best one in the
+// geometric mean and at most 1.53 times as much; counted over all tiles, with a
+// limit of 4.25 whatever the rows, it cost 10.6% and up to 3.8 times.  On 4096
+// slots, us at split 0, 1, ... 6:
+//   4000x37, 1,000 units, 2 rows, 19 shapes    157 240 446 501 589 771 770          takes 0
+//   30x1000, 128 units, 4 rows, 21 shapes      131 119 121 160 259 450 516          takes 2
+//   128x64, 32 units, 4 rows, 1 shape          63 59 55 59 82 130 234               takes 2
+//   64x64, 4 units, 16 rows, 12 shapes         167 137 123 114 112 97 97            takes 6
+//   641x479, 22 units, 218 rows, 65 shapes     2572 1519 1181 978 867 837 757       takes 6
+//   1000x701, 536 units, 20 rows, 104          7046 5182 3885 2964 2405 2313 2861   takes 5
+//   2000x2000, 260 units, 240 rows, 97         14098 8073 5180 3756 2966 3446 4170  takes 4
+//   1500x1200, 470 units, 60 rows, 66          4289 3182 2289 1737 1622 1869 2434   takes 4
+//   512x512, 256 units, 16 rows, 48            1673 1350 1101 921 967 1035 1089     takes 4
+//   1920x1080, 540 units, 60 rows, 4           471 307 364 556 616 765 1016         takes 1
+//   1500x1500, 2,256 units, 16 rows, 10        487 607 623 699 915 922 910          takes 0
+//   512x512, 4,096 units, 1 row, 764           10825 12713 16324 23404 23424 ...    takes 0
+//   1920x1080, 8,160 units, 4 rows, 62         1956 2101 2463 2443 2423 ...         takes 0
 constexpr int kPartsPerSlot = 5;   // bound of the parts per slot, for the retry list
-static int split_units(int n_work, double pixels, double refs, int slots, int capacity)
+static int split_units(int n_work, double pixels, double unit_shapes, int slots, int capacity)
 {
     if (n_work <= 0) return 0;
-    const double rows = pixels / (64.0 * n_work), shapes = 4.0 * refs / n_work;
-    const double crowd = shapes / 40.0;
-    const double fill = std::min(4.25, std::max(0.3, crowd * crowd)) * std::min(1.0, rows / 8.0);
-    const double parts = std::min((double)capacity, slots * fill);
+    const double rows = pixels / (64.0 * n_work), shapes = unit_shapes / n_work;
+    const double most = std::max(1.25, std::min(4.25, 128.0 / rows));
+    const double crowd = std::min(most, (shapes / 34.0) * (shapes / 34.0)) * std::min(1.0, rows / 6.0);
+    const double idle = 0.3 * std::min(std::min(1.0, rows / 8.0), rows * (shapes + 1.0) / 40.0);
+    const double parts = std::min((double)capacity, slots * std::max(crowd, idle));
     int split = 0;
     while (split < 6 && (double)n_work * (double)(2 << split) <= parts) ++split;
     return split;
@@ -447,9 +473,10 @@ static PassBuffers ctx_buffers(gudni_ctx *ctx)
                        ctx->slow_blocks, 256};
 }
 
-// pixels, refs: what the launch covers and how many shape references its
-// tiles hold, for the choice of the split.
-static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, double pixels, double refs)
+// pixels, unit_shapes: what the launch covers and how many shapes its units
+// hold together, for the choice of the split.
+static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, double pixels,
+                         double unit_shapes)
 {
     uint32_t *ctl = b.ctl;
     hipLaunchKernelGGL(dev::reset_counters, dim3(1), dim3(64), 0, ctx->stream, ctl, dev::kCtlWords);
@@ -466,7 +493,7 @@ static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, dou
     f.shape_idx = b.fast_sidx;
     int slog = 0;
     while ((1 << slog) < ctx->spec.max_thresholds) ++slog;
-    f.split = split_units(f.n_work, pixels, refs, 4 * b.fast_blocks, b.retry_capacity);
+    f.split = split_units(f.n_work, pixels, unit_shapes, 4 * b.fast_blocks, b.retry_capacity);
     f.slot_log2 = dev::kFastCapLog2 + 6;
     f.cap_log2 = std::min(dev::kFastCapLog2 + f.split, std::max(slog, dev::kFastCapLog2));
     const int fast_grid = std::max(1, std::min(b.fast_blocks, ((f.n_work << f.split) + 3) / 4));
@@ -486,9 +513,9 @@ static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, dou
     return GUDNI_OK;
 }
 
-static int launch_passes(gudni_ctx *ctx, dev::Frame f, double pixels, double refs)
+static int launch_passes(gudni_ctx *ctx, dev::Frame f, double pixels, double unit_shapes)
 {
-    return launch_passes(ctx, f, ctx_buffers(ctx), pixels, refs);
+    return launch_passes(ctx, f, ctx_buffers(ctx), pixels, unit_shapes);
 }
 
 int read_status(gudni_ctx *ctx)
@@ -747,6 +774,7 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
     cnt.n_tiles = (int32_t)status[1];
     cnt.n_refs = (int32_t)status[2];
     cnt.n_work = (int32_t)status[3];
+    cnt.unit_shapes = status[7];
     return GUDNI_OK;
 }
 
@@ -827,6 +855,7 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
                 cnt[s].n_tiles = (int32_t)st[1];
                 cnt[s].n_refs = (int32_t)st[2];
                 cnt[s].n_work = (int32_t)st[3];
+                cnt[s].unit_shapes = st[7];
             } else if (st[0] == 1 && give_up_pairs > 0) {
                 return 1;
             } else if (st[0] == 1) {
@@ -1136,7 +1165,7 @@ static int run_job(gudni_ctx *ctx, const void *shapes, int32_t n_shapes, const v
         pixels += std::max(0.0, std::min(w, r.box[2]) - (double)r.box[0]) *
                   std::max(0.0, std::min(h, r.box[3]) - (double)r.box[1]);
     }
-    rc = launch_passes(ctx, f, pixels, n_shapes);
+    rc = launch_passes(ctx, f, pixels, (double)unit_shapes((const TileRec *)tiles, work));
     if (rc) return rc;
     rc = read_status(ctx);
     if (rc) return rc;
@@ -1224,7 +1253,7 @@ int gudni_frame_upload(gudni_ctx *ctx, const gudni_jobs *jobs, int32_t width, in
     ctx->frame_h = height;
     ctx->frame_n_work = (int32_t)work.size();
     ctx->frame_n_tiles = v.n_tiles;
-    ctx->frame_n_refs = v.n_refs;
+    ctx->frame_unit_shapes = (double)unit_shapes(tiles.data(), work);
     ctx->frame_index = frame;
     ctx->frame_sort_bits = jobs->j.sort_radix_bits;
     std::memcpy(ctx->background, background, sizeof(ctx->background));
@@ -1256,7 +1285,7 @@ int gudni_frame_render(gudni_ctx *ctx, uint32_t *out_dev, float *out_f32_dev)
         CHECK_HIP(ctx, hipEventRecord(ctx->ev[0], ctx->stream));
     }
     ctx->timed_render = ctx->timing;
-    int rc = launch_passes(ctx, f, (double)ctx->frame_w * ctx->frame_h, ctx->frame_n_refs);
+    int rc = launch_passes(ctx, f, (double)ctx->frame_w * ctx->frame_h, ctx->frame_unit_shapes);
     if (rc) return rc;
     if (ctx->timing) CHECK_HIP(ctx, hipEventRecord(ctx->ev[2], ctx->stream));
     return GUDNI_OK;
@@ -1303,7 +1332,7 @@ int gudni_frame_render_static(gudni_ctx *ctx, uint32_t *out_dev, float *out_f32_
                         reinterpret_cast<float4 *>(base + kOffSlowThr),
                         reinterpret_cast<uint32_t *>(base + kOffSlowHdr),
                         reinterpret_cast<int32_t *>(base + kOffSlowSidx), 1, 64};
-    return launch_passes(ctx, f, b, (double)ctx->frame_w * ctx->frame_h, ctx->frame_n_refs);
+    return launch_passes(ctx, f, b, (double)ctx->frame_w * ctx->frame_h, ctx->frame_unit_shapes);
 }
 
 int gudni_frame_check(gudni_ctx *ctx)
@@ -1375,7 +1404,7 @@ int gudni_scene_bin(gudni_ctx *ctx)
     ctx->frame_h = ctx->scene_h;
     ctx->frame_n_tiles = (int32_t)status[1];
     ctx->scene_n_refs = (int32_t)status[2];
-    ctx->frame_n_refs = (int32_t)status[2];
+    ctx->frame_unit_shapes = cnt.unit_shapes;
     ctx->frame_n_work = (int32_t)status[3];
     ctx->frame_index = 0;
     ctx->frame_sort_bits = ctx->spec.sort_radix_bits;
@@ -1484,7 +1513,7 @@ struct gudni_batch {
     std::vector<int32_t> width, height;
     std::vector<int32_t> work_begin, work_count;
     int32_t n_work = 0;
-    size_t n_refs = 0;         // shape references of all scenes
+    std::vector<uint64_t> unit_shapes;   // per scene: shapes of all its work units
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint64_t captured_gen = 0;     // ctx->scratch_gen the graph was captured with
@@ -1507,6 +1536,7 @@ int gudni_batch_upload(gudni_ctx *ctx, int32_t n_scenes, const gudni_batch_scene
     std::vector<float> bounds;
     std::vector<TileRec> tiles;
     std::vector<int32_t> tile_job, tile_scene, wbegin, wcount;
+    std::vector<uint64_t> unit_sum;
     std::vector<uint32_t> work;
     std::vector<size_t> geo_off, subs_off, pict_off, uses_off, refs_off, frame_off, grads_off;
     std::vector<gudni_gradient> grads;
@@ -1563,6 +1593,7 @@ int gudni_batch_upload(gudni_ctx *ctx, int32_t n_scenes, const gudni_batch_scene
         build_work(ctx->spec, t.data(), v.n_tiles, sc.width, sc.height, w);
         wbegin.push_back((int32_t)work.size());
         wcount.push_back((int32_t)w.size());
+        unit_sum.push_back(unit_shapes(t.data(), w));
         for (uint32_t u : w) work.push_back(u + ((uint32_t)tile_base << 2));
         tiles.insert(tiles.end(), t.begin(), t.end());
         tile_job.insert(tile_job.end(), tj.begin(), tj.end());
@@ -1581,7 +1612,7 @@ int gudni_batch_upload(gudni_ctx *ctx, int32_t n_scenes, const gudni_batch_scene
     b->n_scenes = n_scenes;
     b->device = ctx->device;
     b->n_work = (int32_t)work.size();
-    b->n_refs = refs.size();
+    b->unit_shapes = unit_sum;
     b->frame_off = frame_off;
     b->work_begin = wbegin;
     b->work_count = wcount;
@@ -1792,6 +1823,7 @@ int gudni_batch_upload_outlines(gudni_ctx *ctx, int32_t n_scenes, const gudni_ou
         }
         b->work_begin.push_back((int32_t)(work_used / 4));
         b->work_count.push_back(bc.n_work);
+        b->unit_shapes.push_back(bc.unit_shapes);
         if (e == hipSuccess && bc.n_work) {
             e = append_dev(b->work, work_used, ctx->work.p, 4u * (size_t)bc.n_work, 4, st, off);
             if (e == hipSuccess)
@@ -1809,7 +1841,6 @@ int gudni_batch_upload_outlines(gudni_ctx *ctx, int32_t n_scenes, const gudni_ou
         if (e == hipSuccess && !d->p) e = d->ensure(16);
     if (e != hipSuccess) return hip_fail(e);
     b->n_work = (int32_t)(work_used / 4);
-    b->n_refs = refs_used / 16;
     {
         std::vector<TileRec> th(tiles_used / 32);
         std::vector<int32_t> ts(tiles_used / 32);
@@ -1872,9 +1903,12 @@ static int batch_launch(gudni_ctx *ctx, gudni_batch *b)
     hipLaunchKernelGGL(dev::batch_begin, dim3(blocks), dim3(threads), 0, ctx->stream,
                        (unsigned long long *)b->done.p, b->n_scenes);
     CHECK_HIP(ctx, hipGetLastError());
-    double pixels = 0.0;
-    for (int32_t s = 0; s < b->n_scenes; ++s) pixels += (double)b->width[s] * b->height[s];
-    return launch_passes(ctx, batch_frame(ctx, b), pixels, (double)b->n_refs);
+    double pixels = 0.0, shapes = 0.0;
+    for (int32_t s = 0; s < b->n_scenes; ++s) {
+        pixels += (double)b->width[s] * b->height[s];
+        shapes += (double)b->unit_shapes[s];
+    }
+    return launch_passes(ctx, batch_frame(ctx, b), pixels, shapes);
 }
 
 int gudni_batch_render(gudni_ctx *ctx, gudni_batch *b, int use_graph)
@@ -1937,8 +1971,7 @@ int gudni_batch_render_scene(gudni_ctx *ctx, gudni_batch *b, int32_t scene)
     f.work = (const uint32_t *)b->work.p + b->work_begin[scene];
     f.n_work = b->work_count[scene];
     f.scene_done = nullptr;
-    return launch_passes(ctx, f, (double)b->width[scene] * b->height[scene],
-                         (double)b->n_refs * f.n_work / std::max(1, b->n_work));
+    return launch_passes(ctx, f, (double)b->width[scene] * b->height[scene], (double)b->unit_shapes[scene]);
 }
 
 int gudni_batch_check(gudni_ctx *ctx, gudni_batch *b, float *latency_ms)
