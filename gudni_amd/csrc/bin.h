@@ -38,7 +38,7 @@ struct Workspace {
     int32_t *node_toff = nullptr, *node_roff = nullptr;    // cap_nodes
     int4 *levels = nullptr;        // per level: node begin, node count, pair begin, pair count
     // [0] overflow [1] tiles [2] refs [3] work [4] nodes [5] pairs [6] what
-    // overflowed [7] shapes of all work units (unit_weight)
+    // overflowed, or the level to go on from [7] shapes of all work units (unit_weight)
     uint32_t *status = nullptr;
 };
 
@@ -58,10 +58,10 @@ struct Output {
 // Enqueues the whole binning on `stream`; status[] holds the counts once the
 // stream reaches it (status[0] != 0: nothing valid; 1 = a capacity was
 // exceeded, status[6] bit 0 = nodes, bit 1 = pairs; 2 = the tree is deeper
-// than the level table).
+// than the level table).  from_level > 0: the levels before it are in `w`.
 hipError_t enqueue(const Params &p, const Workspace &w, const ShapeRec *shapes,
                    const float4 *bbox, const float4 *shape_bounds, const Output &out,
-                   hipStream_t stream);
+                   hipStream_t stream, int from_level = 0);
 
 // One scene of a many-scene binning: its parameters, its own workspace and
 // outputs.
@@ -71,7 +71,10 @@ struct SceneJob {
     const ShapeRec *shapes;
     const float4 *bbox, *shape_bounds;
     Output out;
-    int32_t give_up;   // stop with status[0] = 1 as soon as the pairs are seen to outgrow cap_pairs
+    // > 0: stop once all levels together hold more pairs, the next one more than
+    // an eighth of that, or once they hold a quarter and are seen to grow past it;
+    // status[6] is then the next level (and status[0] 0), for enqueue to go on from
+    int32_t stop_pairs;
 };
 
 constexpr int kSceneBlockThreads = 512;

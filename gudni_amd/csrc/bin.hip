@@ -444,16 +444,42 @@ __global__ void __launch_bounds__(kThreads) bin_emit_work(Dev d, WorkFlags f, ui
     emit_work_body(d, f, work, gtid(), gstride());
 }
 
-// Whether the pairs of all levels will outgrow the capacity, after `level` has
-// been advanced: while the next nodes are forced to split or hold cap_shapes
-// shapes on average, a level's pairs grow as this one's did (a shape crosses
-// more cuts the smaller the nodes are, so this is low rather than high).  The
-// first two levels are not asked: their nodes are larger than most shapes.
-__device__ bool outgrows(const Dev &d, int level)
+// Cells of size c (of n in a row) that the box side lo..hi crosses into.
+__device__ __forceinline__ uint32_t cells_crossed(float lo, float hi, float c, int n)
 {
-    if (level < 1 || level + 1 >= d.p.max_levels) return false;
+    const float last = (float)(n - 1);
+    const int a = (int)fminf(fmaxf(floorf(lo / c), 0.0f), last), b = (int)fminf(fmaxf(ceilf(hi / c) - 1.0f, 0.0f), last);
+    return b >= a ? (uint32_t)(b - a + 1) : 1u;
+}
+
+// The pairs of all forced levels together (every thread of the block calls it).
+__device__ uint64_t forced_pairs(const Params &p, const float4 *bbox, int t0, int ts)
+{
+    uint64_t mine = 0, total;
+    for (int s = t0; s < p.n_shapes; s += ts) {
+        const float4 bb = bbox[s];
+        uint32_t x = 1, y = 1;
+        mine += 1;
+        for (int k = 1; k <= p.canvas_depth - p.tile_depth; ++k) {
+            const float c = (float)(1 << (p.canvas_depth - k));
+            y = cells_crossed(bb.y, bb.w, c, 1 << k);
+            mine += x * y;
+            x = cells_crossed(bb.x, bb.z, c, 1 << k);
+            mine += x * y;
+        }
+    }
+    (void)devscan::block_excl_scan(mine, total);
+    return total;
+}
+
+// Whether the pairs are seen, after `level` has been advanced, to grow to more
+// than twice `most`: while the next nodes are forced to split or hold cap_shapes
+// shapes on average, a level's pairs are taken to grow as this one's did.  The
+// first two levels are not asked: their nodes are larger than most shapes.
+__device__ bool outgrows(const Dev &d, int level, int most)
+{
     const int4 lv = d.levels[level], nx = d.levels[level + 1];
-    if (lv.w == 0) return false;
+    if (level < 1 || lv.w == 0) return false;
     const float grow = (float)nx.w / (float)lv.w;
     float nodes = (float)nx.y, pairs = (float)nx.w, total = (float)(nx.z + nx.w);
     const int forced = 2 * (d.p.canvas_depth - d.p.tile_depth), last = 2 * (d.p.canvas_depth - 3);
@@ -462,7 +488,7 @@ __device__ bool outgrows(const Dev &d, int level)
         pairs *= grow;
         total += pairs;
     }
-    return total > (float)d.cap_pairs;
+    return total > 2.0f * (float)most;
 }
 
 // One scene per block: the steps of enqueue() in order, with block barriers
@@ -490,6 +516,11 @@ __global__ void __launch_bounds__(kSceneBlockThreads) bin_scene_block(const Scen
     const int t0 = (int)threadIdx.x, ts = (int)blockDim.x;
     init_body(d, t0, ts);
     __syncthreads();
+    // a tree with more than stop_pairs pairs in its forced levels alone; those of n
+    // shapes hold at most 2 n 4^(canvas - tile depth)
+    const int side = max(0, d.p.canvas_depth - d.p.tile_depth);
+    const bool large = j.stop_pairs && ((int64_t)d.p.n_shapes << (2 * side + 1)) > j.stop_pairs &&
+                       forced_pairs(d.p, j.bbox, t0, ts) > (uint64_t)j.stop_pairs;
     int depth = d.p.max_levels;
     for (int l = 0; l < d.p.max_levels; ++l) {
         decide_body(d, j.shapes, l, t0, ts);
@@ -501,9 +532,11 @@ __global__ void __launch_bounds__(kSceneBlockThreads) bin_scene_block(const Scen
         __syncthreads();
         if (t0 == 0) {
             advance_body(d, l);
-            if (j.give_up && !d.status[0] && outgrows(d, l)) {
-                d.status[6] = 2u;
-                d.status[0] = 1u;
+            if (j.stop_pairs && !d.status[0] && l + 1 < d.p.max_levels) {
+                const int next = d.levels[l + 1].w, pairs = d.levels[l + 1].z + next;
+                if ((pairs > j.stop_pairs && next > j.stop_pairs / 8) ||
+                    (pairs > j.stop_pairs / 4 && (large || outgrows(d, l, j.stop_pairs))))
+                    d.status[6] = (uint32_t)(l + 1);
             }
         }
         __syncthreads();
@@ -511,6 +544,7 @@ __global__ void __launch_bounds__(kSceneBlockThreads) bin_scene_block(const Scen
         __syncthreads();
         scatter_body(d, j.bbox, l, t0, ts);
         __syncthreads();
+        if (!d.status[0] && d.status[6]) return;   // the same for every thread of the block
         // the levels below a level without nodes are empty: their steps
         // would do nothing (the same for every thread of the block)
         if (d.status[0] || l + 1 >= d.p.max_levels || d.levels[l + 1].y == 0) {
@@ -586,7 +620,7 @@ void carve(Workspace &w, void *base, int32_t cap_pairs, int32_t cap_nodes, int32
 }
 
 hipError_t enqueue(const Params &p, const Workspace &w, const ShapeRec *shapes, const float4 *bbox,
-                   const float4 *shape_bounds, const Output &out, hipStream_t stream)
+                   const float4 *shape_bounds, const Output &out, hipStream_t stream, int from_level)
 {
     Dev d;
     d.p = p;
@@ -606,8 +640,8 @@ hipError_t enqueue(const Params &p, const Workspace &w, const ShapeRec *shapes, 
     d.cap_pairs = w.cap_pairs;
     d.cap_nodes = w.cap_nodes;
     const dim3 g(kBlocks), b(kThreads);
-    hipLaunchKernelGGL(bin_init, g, b, 0, stream, d);
-    for (int l = 0; l < p.max_levels; ++l) {
+    if (from_level == 0) hipLaunchKernelGGL(bin_init, g, b, 0, stream, d);
+    for (int l = from_level; l < p.max_levels; ++l) {
         hipLaunchKernelGGL(bin_decide, g, b, 0, stream, d, shapes, l);
         SplitFlags sf{w.levels, w.node_meta, l, 0, 0};
         devscan::excl_scan(sf, w.partials, d.node_scan, stream);

@@ -183,9 +183,7 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
 // The same for n scenes at once, one block per scene (for scenes of a few
 // thousand shapes, where the per-level launches of bin_scene cost more than
 // the work): one launch and one synchronisation while the capacities hold.
-// give_up_pairs > 0: a scene that has or will have more (node, shape) pairs
-// than that is not built; returns 1 then.
-int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n, int32_t give_up_pairs = 0);
+int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n);
 // Bounds-checks shape records (and tiles) against the common buffers and
 // fills each shape's strand extent (xmin, ymin, xmax, ymax).
 int validate_job(gudni_ctx *ctx, const CommonView &cv, const ShapeRec *shapes, int32_t n_shapes,

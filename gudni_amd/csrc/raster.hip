@@ -673,20 +673,21 @@ int validate_job(gudni_ctx *ctx, const CommonView &cv, const ShapeRec *shapes,
     return GUDNI_OK;
 }
 
-// Whether one block builds a scene's tree sooner than the level launches,
-// which cost 0.6 to 0.9 ms (some 200 of them) however little there is to do.
-// `cells`: the root's forced leaves.  The block's time goes with the pairs it
-// moves, at most shapes x cells a level.  Measured (us, block against
-// launches): 250^2, 120 shapes, 16-px tiles (256 cells) 130 / 569; 640^2, 300,
-// 256 px (16) 108 / 825; 512^2, 1,000, 32 px (256) 344 / 675; 800^2, 3,000,
-// 256 px (16) 529 / 823; 1920^2, 1,000, 64 px (1,024) 764 / 963; beyond the
-// line 512^2, 2,000, 16 px (1,024) 1,047 / 685.  Large shapes reach most
-// tiles of a deep tree (580 scribbles on 102x462: 1.4M references, 15 ms in
-// one block): a build that passes its first capacity of pairs, or is seen to
-// grow past it (outgrows), gives up and goes to the launches.  Every scene is
-// tried alike, whatever the context built before.  Giving up costs 40 us (1,000
-// scribbles on 512^2: 790 us in all, 742 by the launches alone; 1,100 where the
-// block filled its capacity first).
+// Whether one block begins a scene's tree (bin_scene_block), which the level
+// launches take 0.45 to 0.9 ms for (some 200 of them) however little there is to
+// do.  `cells`: the root's forced leaves.  The block's time goes with the pairs it
+// moves: it builds trees of about kBlockPairs whole and stops at larger ones (a
+// quarter of the way where it foresees them), whose remaining levels are launched
+// from where it stopped, so that its levels are not built twice.  Every scene is
+// begun alike, whatever the context built before.  scene_bin, us, by the launches
+// alone and now:
+//   built whole    250^2, 120 shapes, 16-px tiles 398 / 127; 640^2, 300, 256 px 563
+//                  / 107; 512^2, 1,000, 32 px 456 / 251; 800^2, 3,000, 256 px 654 /
+//                  352; 640^2, 300, 32 px 578 / 373; 400^2, 4,000, 64 px 644 / 476
+//   foreseen       512^2, 1,000, 16 px 466 / 409; 1920^2, 1,000, 64 px 638 / 594;
+//                  1,000 scribbles on 512^2 (3.1M references) 712 / 719; 400 on
+//                  256^2 492 / 457; 580 on 462^2 717 / 618
+//   not foreseen   400^2, 4,000, 32 px 583 / 587
 constexpr int32_t kBlockPairs = 1 << 16;
 static bool one_block_scene(int64_t shapes, int64_t cells)
 {
@@ -695,25 +696,6 @@ static bool one_block_scene(int64_t shapes, int64_t cells)
 
 int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt)
 {
-    const int side = ceil_log2(std::max(in.width, in.height)) -
-                     ceil_log2(in.max_tile_size > 0 ? in.max_tile_size : ctx->spec.max_tile_size);
-    if (one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side))) {
-        if (ctx->timing) {
-            for (hipEvent_t &e : ctx->bin_ev)
-                if (!e) CHECK_HIP(ctx, hipEventCreate(&e));
-            CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[0], ctx->stream));
-        }
-        const int rc = bin_scenes(ctx, &in, &out, &cnt, 1, kBlockPairs);
-        if (rc < 0) return rc;
-        if (rc == GUDNI_OK) {
-            if (ctx->timing) {
-                CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[1], ctx->stream));
-                CHECK_HIP(ctx, hipEventSynchronize(ctx->bin_ev[1]));
-                CHECK_HIP(ctx, hipEventElapsedTime(&ctx->last_bin_ms, ctx->bin_ev[0], ctx->bin_ev[1]));
-            }
-            return GUDNI_OK;
-        }
-    }
     binning::Params bp;
     bp.n_shapes = in.n_shapes;
     bp.canvas_depth = ceil_log2(std::max(in.width, in.height));
@@ -730,6 +712,7 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
     // so the deepest level is 2 (cd - 3).  One level more for margin (a
     // deeper tree stops with an error, never silently).
     bp.max_levels = std::max(2, 2 * (bp.canvas_depth - 3) + 2);
+    const int side = bp.canvas_depth - bp.tile_depth;
     if (!ctx->bin_cap_pairs) {
         ctx->bin_cap_pairs = (int32_t)std::min<int64_t>(std::max<int64_t>(1 << 16, 8 * (int64_t)bp.n_shapes), 1 << 28);
         ctx->bin_cap_nodes = std::max(1 << 15, bp.n_shapes / 4);
@@ -751,10 +734,20 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
         binning::Output o{(TileRec *)out.tiles->p, (int32_t *)out.tile_job->p, (ShapeRec *)out.refs->p,
                           (float4 *)out.ref_bounds->p, (uint32_t *)out.work->p};
         if (ctx->timing) CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[0], ctx->stream));
-        CHECK_HIP(ctx, binning::enqueue(bp, ws, in.shapes, in.bbox, in.bounds, o, ctx->stream));
+        const bool block = one_block_scene(in.n_shapes, side <= 0 ? 1 : (int64_t)1 << (2 * side));
+        if (block) {
+            const binning::SceneJob job{bp, ws, in.shapes, in.bbox, in.bounds, o, kBlockPairs};
+            CHECK_HIP(ctx, upload(ctx, ctx->bins_jobs, &job, sizeof(job)));
+            CHECK_HIP(ctx, binning::enqueue_scenes((const binning::SceneJob *)ctx->bins_jobs.p, 1, ctx->stream));
+            CHECK_HIP(ctx, hipMemcpyAsync(status, ws.status, sizeof(status), hipMemcpyDeviceToHost, ctx->stream));
+            CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        }
+        const int from_level = block && status[0] == 0 ? (int)status[6] : 0;
+        if (!block || from_level > 0) {
+            CHECK_HIP(ctx, binning::enqueue(bp, ws, in.shapes, in.bbox, in.bounds, o, ctx->stream, from_level));
+            CHECK_HIP(ctx, hipMemcpyAsync(status, ws.status, sizeof(status), hipMemcpyDeviceToHost, ctx->stream));
+        }
         if (ctx->timing) CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[1], ctx->stream));
-        CHECK_HIP(ctx, hipMemcpyAsync(status, ws.status, sizeof(status), hipMemcpyDeviceToHost,
-                                      ctx->stream));
         CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (status[0] == 0) break;
         if (status[0] != 1)
@@ -778,7 +771,7 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
     return GUDNI_OK;
 }
 
-int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n, int32_t give_up_pairs)
+int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cnt, int n)
 {
     if (n <= 0) return GUDNI_OK;
     std::vector<binning::Params> params((size_t)n);
@@ -805,7 +798,6 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
         // count per tile, and tiles never outnumber nodes
         cap_pairs[s] = (int32_t)std::max<int64_t>(
             std::min<int64_t>(std::max<int64_t>(1 << 14, 8 * (int64_t)bp.n_shapes), 1 << 28), cap_nodes[s]);
-        if (give_up_pairs > 0) cap_pairs[s] = std::max(give_up_pairs, cap_nodes[s]);
     }
     std::vector<int> todo((size_t)n);
     for (int s = 0; s < n; ++s) todo[s] = s;
@@ -837,7 +829,7 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
             j.shapes = in[s].shapes;
             j.bbox = in[s].bbox;
             j.shape_bounds = in[s].bounds;
-            j.give_up = give_up_pairs > 0 ? 1 : 0;
+            j.stop_pairs = 0;
             j.out = binning::Output{(TileRec *)o.tiles->p, (int32_t *)o.tile_job->p, (ShapeRec *)o.refs->p,
                                     (float4 *)o.ref_bounds->p, (uint32_t *)o.work->p};
         }
@@ -856,8 +848,6 @@ int bin_scenes(gudni_ctx *ctx, const BinIn *in, const BinOut *out, BinCounts *cn
                 cnt[s].n_refs = (int32_t)st[2];
                 cnt[s].n_work = (int32_t)st[3];
                 cnt[s].unit_shapes = st[7];
-            } else if (st[0] == 1 && give_up_pairs > 0) {
-                return 1;
             } else if (st[0] == 1) {
                 // grow only what ran out; fail once it is at its clamp
                 const bool over_nodes = (st[6] & 1u) != 0, over_pairs = (st[6] & 2u) != 0;

@@ -59,3 +59,42 @@ def test_binning_does_not_depend_on_the_scene_before():
     finally:
         r.close()
     assert np.median(after_small) <= 1.2 * np.median(after_big)
+
+
+@pytest.mark.parametrize("tile", [16, 32, 64, 256])
+@pytest.mark.parametrize("make", [lambda: S.batch_scene(400, 4000, 4000), lambda: S.batch_scene(1000, 4000, 4000),
+                                  lambda: S.batch_scene(1920, 1000, 1000), lambda: S.uniform_512(60, 700, 1),
+                                  lambda: S.batch_scene(400, 4097, 4000), lambda: S.batch_scene(20, 4000, 1)])
+def test_tree_goes_on_where_the_block_stops(make, tile):
+    """Trees that the block builds whole, stops at early, stops at late, and does
+    not begin (more than 4,096 shapes)."""
+    spec = G.default_spec(max_tile_size=tile)
+    r = G.Rasterizer(spec)
+    try:
+        compare_binning(r, make(), spec)
+    finally:
+        r.close()
+
+
+def test_the_last_level_is_not_given_up():
+    """4,000 shapes on 400^2 in 64-px tiles come to 66,304 pairs in a block's hands,
+    2,982 of them in the last level; 4,097 are built by the level launches alone.
+    The ratio of the medians is about 1, and was 2 where the block gave up there
+    and the launches began anew."""
+    rs, times = [], []
+    for n in (4000, 4097):
+        r = G.Rasterizer(G.default_spec(max_tile_size=64))
+        r.scene_upload_outlines(S.batch_scene(400, n, 4000))
+        rs.append(r)
+        times.append([])
+    try:
+        for k in range(25):
+            for r, t in zip(rs, times):
+                start = time.perf_counter()
+                r.scene_bin()
+                if k >= 5:
+                    t.append(time.perf_counter() - start)
+    finally:
+        for r in rs:
+            r.close()
+    assert np.median(times[0]) <= 1.35 * np.median(times[1]), [np.median(t) for t in times]
