@@ -1328,6 +1328,25 @@ int check_scene(gudni_ctx *ctx, const gudni_adjoint_batch::Scene &sc, int s)
 
 int fill_descs(gudni_ctx *ctx, gudni_adjoint_batch *a);
 
+// Blocks of the pass over n_work units.
+int pass_blocks(const gudni_adjoint_batch *a, int32_t n_work)
+{
+    return std::max(1, std::min(a->blocks, (n_work + 3) / 4));
+}
+
+// The colour stream (256 KB a wave slot, 0.5 GB for a full chip) of the slots that
+// the batch's units can fill.  Their number changes with the parameters, so it
+// is rounded up to a power of two: the stream seldom grows while a scene is fitted.
+// No launch is in flight.
+int ensure_stream(gudni_ctx *ctx, gudni_adjoint_batch *a)
+{
+    int blocks = 1;
+    while (blocks < pass_blocks(a, a->n_work)) blocks *= 2;
+    blocks = std::min(blocks, a->blocks);
+    CHECK_HIP(ctx, a->cols_fast.ensure((size_t)blocks * 4 * adj::kStream * 64 * 16));
+    return GUDNI_OK;
+}
+
 // Serialises, bins and validates every scene, then (re)uploads all buffers
 // but the targets.
 int build(gudni_ctx *ctx, gudni_adjoint_batch *a)
@@ -1451,8 +1470,9 @@ int build(gudni_ctx *ctx, gudni_adjoint_batch *a)
     CHECK_HIP(ctx, a->copy_hdr.ensure(fast_slots * ((size_t)1 << dev::kFastCapLog2) * 64 * 4));
     CHECK_HIP(ctx, a->ends_fast.ensure(fast_slots * ((size_t)1 << dev::kFastCapLog2) * 4 * 64 * 16));
     CHECK_HIP(ctx, a->orig_slow.ensure(slow_slots * scap * 2 * 64 * 16));
-    CHECK_HIP(ctx, a->cols_fast.ensure(fast_slots * adj::kStream * 64 * 16));
     CHECK_HIP(ctx, a->cols_slow.ensure(slow_slots * adj::kStream * 64 * 16));
+    rc = ensure_stream(ctx, a);
+    if (rc) return rc;
     CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return GUDNI_OK;
 }
@@ -1629,6 +1649,8 @@ int assemble(gudni_ctx *ctx, gudni_adjoint_batch *a)
     a->n_work = (int32_t)wb;
     int rc = ensure_control(ctx, a->n_work);
     if (rc) return rc;
+    rc = ensure_stream(ctx, a);
+    if (rc) return rc;
     return fill_descs(ctx, a);
 }
 
@@ -1746,7 +1768,7 @@ int launch(gudni_ctx *ctx, gudni_adjoint_batch *a, int32_t work_begin, int32_t n
     af.copy_hdr = (uint32_t *)a->copy_hdr.p;
     af.q_ends = (float4 *)a->ends_fast.p;
     af.q_cols = (float4 *)a->cols_fast.p;
-    const int grid = std::max(1, std::min(a->blocks, (n_work + 3) / 4));
+    const int grid = pass_blocks(a, n_work);
     hipLaunchKernelGGL(adj::adjoint_pass, dim3(grid), dim3(256), 0, st, af, 0);
     CHECK_HIP(ctx, hipGetLastError());
     int slog = 0;
