@@ -105,13 +105,12 @@ struct AdjFrame {
     float4 *q_cols;               // [slots][kStream][64]: the colours of each lane's first sections
 };
 
-// Section colours that a lane keeps from the forward sweep for the backward,
-// which also keeps the colours of its listed sections there, in the row of
-// each one's number among them.  That row's forward colour has been read (a
-// section is listed after it is swept), and no section that still waits in the
-// list has it (a list holds fewer sections than there are rows).
+// Section colours that a lane keeps from the forward sweep for the backward.  A
+// section's row is its number modulo kStream; the backward sweep writes the rows
+// of sections past the first kStream that it lists, and walks its list before a
+// lane gets to a section whose row a listed one still has.
 constexpr int kStream = 256;
-static_assert(kSections < kStream && kStream <= 256, "a list entry names its row with 8 bits");
+static_assert(kStream <= 256, "a list entry names its row with 8 bits");
 
 enum Mode { kRecord = 0, kApply = 1 };
 
@@ -862,9 +861,9 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
     Sweep p;
     start_sweep(p, st);
     int guard = (int)kSectionGuard;
-    // sections swept and sections listed: seq numbers the forward's rows,
-    // listed the rows that hold listed sections' colours
-    uint32_t status = 0, row = 0, seq = 0, listed = 0;
+    // sections swept, and the next whose row is that of a listed one
+    constexpr uint32_t kNever = ~0u;
+    uint32_t status = 0, row = 0, seq = 0, taken = kNever;
     bool alive = ok && p.pixel_y <= c.float_height;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 G = alive ? d.gpix[(long long)c.dy * s.width + c.dx] : zero;
@@ -973,10 +972,10 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                     }
                     have = G.x * area != 0.0f || G.y * area != 0.0f || G.z * area != 0.0f || G.w * area != 0.0f;
                     if (have) {
-                        const uint32_t k = listed & (uint32_t)(kStream - 1);
-                        if (listed != seq || seq >= (uint32_t)kStream) cols[k * kWave] = col;
+                        const uint32_t k = seq & (uint32_t)(kStream - 1);
+                        if (seq >= (uint32_t)kStream) cols[k * kWave] = col;
                         at = (uint32_t)lane | (row << 6) | (k << 24);
-                        ++listed;
+                        taken = min(taken, seq + (uint32_t)kStream);
                     }
                     ++seq;
                     s0 = st.s0;
@@ -996,7 +995,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
         }
         const uint64_t mask = __ballot(have);
         const int n = __popcll(mask);
-        if (count + n > kSections || !running) {
+        if (count + n > kSections || !running || __any(seq == taken)) {
             __threadfence_block();   // colours kept by other lanes
             wave_sync();
             for (int e0 = 0; e0 < count; e0 += kWave) {
@@ -1022,6 +1021,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
             }
             wave_sync();
             count = 0;
+            taken = have ? seq - 1u + (uint32_t)kStream : kNever;
             if (!running) break;
         }
         if (have) {
