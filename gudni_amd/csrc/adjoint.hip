@@ -1039,7 +1039,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
 // One work unit, phases A-D.  It and the stages it calls (generation, both
 // sweeps, the line map) are inlined into the kernel: a call would take the
 // frame, the scene descriptor and the queues by address, which keeps them in
-// per-lane scratch memory for the whole unit (848 bytes a lane, against 320
+// per-lane scratch memory for the whole unit (848 bytes a lane, against 288
 // inlined).
 template <bool kCompact>
 __device__ __forceinline__ void adj_unit(const Frame &f, const AdjDesc &d, int lane, uint32_t unit, Queue &q,
@@ -1573,9 +1573,9 @@ int device_serialize_scenes(gudni_ctx *ctx, gudni_adjoint_batch *a, const std::v
     return GUDNI_OK;
 }
 
-// Bins the listed scenes' serialised shapes: one scene with the device-wide
-// level launches (a whole GPU on one tree), several in one launch of a block
-// per scene (the level launches would cost more than the work).
+// Bins the listed scenes' serialised shapes: one scene as a frame's (bin_scene: a
+// block, and device-wide level launches for what outgrows it), several in one
+// launch of a block per scene (the level launches would cost more than the work).
 int device_bin_scenes(gudni_ctx *ctx, gudni_adjoint_batch *a, const std::vector<int> &which)
 {
     const size_t n = which.size();

@@ -23,7 +23,9 @@
 // arguments as CallKernels.hs:254 passes them) and the reversed job numbering
 // of queueRasterJobs (CallKernels.hs:241, 255).  Every kernel is grid-stride
 // over counts it reads from device memory, so the whole build is enqueued
-// without a host round trip; capacities are checked on the device.
+// without a host round trip; capacities are checked on the device.  A small tree
+// is built by one block in one launch, and a tree that the block leaves is built on
+// by these kernels from the level it stopped at, with one round trip between.
 #include "bin.h"
 #include "scan.h"
 

@@ -879,10 +879,10 @@ __device__ void sort_queue(Queue &q)
 // insertion sort then only meets inversions inside a bucket.  Both steps
 // are stable, so the permutation is the stable sort's, i.e. the reference's
 // bubble sort's.  The 64 lanes of a wave sort their 64 columns in lockstep;
-// `hist` is the lane's column of a [32][64] u16 table (the tile table's
-// colour cache, which is rebuilt after the sort).  Columns with fewer than
-// kRadixMin records, or more than half a ring, take the insertion sort
-// alone.
+// `hist` is the lane's column of a [32][64] u16 table (the tile table's, in
+// the place of generation's strands and the sweep's sections).  Columns with
+// fewer than kRadixMin records, or more than half a ring, take the insertion
+// sort alone.
 constexpr int kRadixMin = 8;
 
 __device__ __forceinline__ int top_digit(float top, float scale, int nb)
