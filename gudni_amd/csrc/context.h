@@ -95,6 +95,7 @@ struct gudni_ctx {
     float last_ser_ms = 0;
     // timing
     bool timing = false, timed_render = false, timed_adjoint = false;
+    int32_t timed_split = 0;      // of the timed render's launch (split_units)
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     float last_ms[2] = {0, 0};
     unsigned long long last_cycles[8] = {0, 0, 0, 0, 0, 0, 0, 0};

@@ -1802,8 +1802,6 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
     const bool active = init_column(f, s, t, job, column, c) && mine;
     const int dslot = tile * f.threads_per_tile + column;
     const bool timed = f.stage_cycles != nullptr;
-    // a unit counts once, however many waves run it
-    if (timed && lane == 0 && part == 0) atomicAdd(f.stage_cycles + 3, 1ull);
     const long long t0 = timed ? clock64() : 0;
     if (kCompact) {
         // the tile's tags and solid colours, by tile-local index
@@ -1896,6 +1894,7 @@ __device__ __forceinline__ void run_unit(const Frame &f, const SceneDesc &s, int
             atomicAdd(f.stage_cycles + 0, (unsigned long long)(t1 - t0));
             atomicAdd(f.stage_cycles + 1, (unsigned long long)(t2 - t1));
             atomicAdd(f.stage_cycles + 2, (unsigned long long)(t3 - t2));
+            atomicAdd(f.stage_cycles + 3, 1ull);   // parts; units once read (gudni_frame_check)
         }
     }
 }

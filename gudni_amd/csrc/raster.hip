@@ -494,6 +494,7 @@ static int launch_passes(gudni_ctx *ctx, dev::Frame f, const PassBuffers &b, dou
     int slog = 0;
     while ((1 << slog) < ctx->spec.max_thresholds) ++slog;
     f.split = split_units(f.n_work, pixels, unit_shapes, 4 * b.fast_blocks, b.retry_capacity);
+    if (ctx->timed_render) ctx->timed_split = f.split;
     f.slot_log2 = dev::kFastCapLog2 + 6;
     f.cap_log2 = std::min(dev::kFastCapLog2 + f.split, std::max(slog, dev::kFastCapLog2));
     const int fast_grid = std::max(1, std::min(b.fast_blocks, ((f.n_work << f.split) + 3) / 4));
@@ -1338,6 +1339,7 @@ int gudni_frame_check(gudni_ctx *ctx)
         ctx->last_ms[1] = b;
         CHECK_HIP(ctx, hipMemcpy(ctx->last_cycles, ctx->cycles.p, sizeof(ctx->last_cycles),
                                  hipMemcpyDeviceToHost));
+        ctx->last_cycles[3] >>= ctx->timed_split;   // a unit counts once, however many waves ran it
         ctx->timed_render = false;
     }
     return GUDNI_OK;
