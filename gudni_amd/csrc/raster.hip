@@ -744,12 +744,13 @@ int bin_scene(gudni_ctx *ctx, const BinIn &in, const BinOut &out, BinCounts &cnt
             CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
         }
         const int from_level = block && status[0] == 0 ? (int)status[6] : 0;
-        if (!block || from_level > 0) {
+        const bool launches = !block || from_level > 0;
+        if (launches) {
             CHECK_HIP(ctx, binning::enqueue(bp, ws, in.shapes, in.bbox, in.bounds, o, ctx->stream, from_level));
             CHECK_HIP(ctx, hipMemcpyAsync(status, ws.status, sizeof(status), hipMemcpyDeviceToHost, ctx->stream));
         }
         if (ctx->timing) CHECK_HIP(ctx, hipEventRecord(ctx->bin_ev[1], ctx->stream));
-        CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (launches || ctx->timing) CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (status[0] == 0) break;
         if (status[0] != 1)
             return set_error(ctx, GUDNI_ERR_ARG, "scene binning: tile tree deeper than the canvas allows");
