@@ -107,8 +107,11 @@ struct AdjFrame {
 
 // Section colours that a lane keeps from the forward sweep for the backward.  A
 // section's row is its number modulo kStream; the backward sweep writes the rows
-// of sections past the first kStream that it lists, and walks its list before a
-// lane gets to a section whose row a listed one still has.
+// of sections past the first kStream.  A lane sweeps at most one section a step,
+// and the wave walks its list at the latest kStream - 1 steps after it last did:
+// no listed section's row is written again before that.  (Following each lane's
+// oldest listed section instead cost 1.5% of a fit's step, rows of their own for
+// listed sections 3 to 4%; a step counter costs nothing measurable.)
 constexpr int kStream = 256;
 static_assert(kStream <= 256, "a list entry names its row with 8 bits");
 
@@ -861,9 +864,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
     Sweep p;
     start_sweep(p, st);
     int guard = (int)kSectionGuard;
-    // sections swept, and the next whose row is that of a listed one
-    constexpr uint32_t kNever = ~0u;
-    uint32_t status = 0, row = 0, seq = 0, taken = kNever;
+    uint32_t status = 0, row = 0, seq = 0;
     bool alive = ok && p.pixel_y <= c.float_height;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 G = alive ? d.gpix[(long long)c.dy * s.width + c.dx] : zero;
@@ -877,7 +878,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
     float e_top = 0.0f, e_bot = 0.0f;
     bool span_open = false, pend = false;
     int pend_org = -1, pend_end = 0, cur_org = -1, cur_end = 0;
-    int count = 0;
+    int count = 0, steps = 0;   // listed sections; steps since the list was walked
     for (;;) {
         const bool running = __any(alive);
         const bool border = alive && p.sx1 == 1.0f && p.sy1 < p.pixel_y;
@@ -885,7 +886,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
         bool have = false;
         float area = 0.0f;
         uint64_t s0 = 0, s1 = 0;
-        uint32_t at = 0;
+        const uint32_t at = (uint32_t)lane | (row << 6) | ((seq & (uint32_t)(kStream - 1)) << 24);
         if (alive && (advance || !border)) {
             if (!((p.sx1 < 1.0f) || (p.sy1 < p.pixel_y))) {
                 // the pixel's end; the span state starts afresh
@@ -936,8 +937,13 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                     p.sx0 = p.sx1;
                     p.sx1 = nx;
                     float4 col;
-                    if (seq < (uint32_t)kStream) col = cols[seq * kWave];
-                    else col = determine_color<kCompact>(f, s, st, sidx, tt, c.dx, c.dy + (int)row);
+                    if (seq < (uint32_t)kStream) {
+                        col = cols[seq * kWave];
+                    } else {
+                        col = determine_color<kCompact>(f, s, st, sidx, tt, c.dx, c.dy + (int)row);
+                        cols[(seq & (uint32_t)(kStream - 1)) * kWave] = col;
+                    }
+                    ++seq;
                     const float dy = p.sy1 - p.sy0;
                     area = (p.sx1 - p.sx0) * dy;
                     float et = 1.0f, eb = 1.0f;
@@ -971,13 +977,6 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
                         }
                     }
                     have = G.x * area != 0.0f || G.y * area != 0.0f || G.z * area != 0.0f || G.w * area != 0.0f;
-                    if (have) {
-                        const uint32_t k = seq & (uint32_t)(kStream - 1);
-                        if (seq >= (uint32_t)kStream) cols[k * kWave] = col;
-                        at = (uint32_t)lane | (row << 6) | (k << 24);
-                        taken = min(taken, seq + (uint32_t)kStream);
-                    }
-                    ++seq;
                     s0 = st.s0;
                     s1 = st.s1;
                     if (crossing) {
@@ -995,7 +994,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
         }
         const uint64_t mask = __ballot(have);
         const int n = __popcll(mask);
-        if (count + n > kSections || !running || __any(seq == taken)) {
+        if (count + n > kSections || !running || ++steps == kStream - 1) {
             __threadfence_block();   // colours kept by other lanes
             wave_sync();
             for (int e0 = 0; e0 < count; e0 += kWave) {
@@ -1021,7 +1020,7 @@ __device__ __forceinline__ uint32_t sweep_backward(const Frame &f, const AdjDesc
             }
             wave_sync();
             count = 0;
-            taken = have ? seq - 1u + (uint32_t)kStream : kNever;
+            steps = 0;
             if (!running) break;
         }
         if (have) {
